@@ -351,7 +351,10 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     xvo[q] = (m < M && xpi[q] >= 0) ? (uint32_t)(src.xoff(m) + xpk[q]) * 2u : 0x80000000u;
   }
 
-  auto load = [&](Stage& s, int t, bool live) {
+  // tail: the ragged step, whose rows end inside it: its ranges end with the
+  // tile's last row (the matrix may end there, and memory with it), and its
+  // scales are read one by one, as no wider load is sure to end where they do
+  auto load = [&](Stage& s, int t, bool live, bool tail = false) {
     if constexpr (XM > 0 && !XRES) {
       const uint32_t xstep = (uint32_t)t * STEPK * 2;
       const auto rx = make_rsrc(reinterpret_cast<const char*>(src.x) + xstep,
@@ -362,7 +365,9 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     }
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
-      const auto rw = make_rsrc(tl.w[j] + (int64_t)t * STEPB, live ? w_nrec[j] : 0u);
+      uint32_t wn = w_nrec[j];
+      if (tail && wn) wn -= (uint32_t)(t + 1) * STEPB - rowB;
+      const auto rw = make_rsrc(tl.w[j] + (int64_t)t * STEPB, live ? wn : 0u);
 #pragma unroll
       for (int L = 0; L < NL; ++L)
         s.w[j][L] = __builtin_amdgcn_raw_buffer_load_b128(rw, wofs + L * 64, 0, 0);
@@ -370,9 +375,22 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     if constexpr (!SBL) {
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        const auto rs = make_rsrc(tl.s[j] + (int64_t)t * STEPG * 2, live ? s_nrec[j] : 0u);
-        const auto rb = make_rsrc(tl.b[j] + (int64_t)t * STEPG * 2, live ? s_nrec[j] : 0u);
-        if constexpr (NSV == 2) {
+        uint32_t sn = s_nrec[j];
+        if (tail && sn) sn -= (uint32_t)(t + 1) * (STEPG * 2) - sRowB;
+        const auto rs = make_rsrc(tl.s[j] + (int64_t)t * STEPG * 2, live ? sn : 0u);
+        const auto rb = make_rsrc(tl.b[j] + (int64_t)t * STEPG * 2, live ? sn : 0u);
+        if (tail) {
+#pragma unroll
+          for (int v = 0; v < NSV; ++v) {
+            auto two = [&](__amdgpu_buffer_rsrc_t d) {
+              const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b16(d, sofs + 4 * v, 0, 0);
+              const uint32_t hi = __builtin_amdgcn_raw_buffer_load_b16(d, sofs + 4 * v + 2, 0, 0);
+              return lo | hi << 16;
+            };
+            s.s[j][v] = two(rs);
+            s.b[j][v] = two(rb);
+          }
+        } else if constexpr (NSV == 2) {
           const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(rs, sofs, 0, 0);
           const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(rb, sofs, 0, 0);
           s.s[j][0] = a[0]; s.s[j][1] = a[1]; s.b[j][0] = q[0]; s.b[j][1] = q[1];
@@ -653,7 +671,7 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     // ---- ragged tail: at most one step; groups past K are zeroed ----------
     if (fe < se) {
       Stage s;
-      load(s, fe, true);
+      load(s, fe, true, true);
 #pragma unroll
       for (int j = 0; j < TJ; ++j)
 #pragma unroll
