@@ -49,6 +49,10 @@ UNITS = [("abi.hip", []), ("formats.hip", []), ("prep.hip", []), ("route.hip", [
     ("inst.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}"] + glu)
     for glu in ([], ["-DMQ_INST_GLU"]) for dt in (0, 1) for bits in (4, 8)
 ] + [
+    # the wide kernel's instruction order (dense.hip)
+    ("dense.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}", "-fno-slp-vectorize"])
+    for dt in (0, 1) for bits in (4, 8)
+] + [
     # the quad kernel keeps its MFMA accumulators in VGPRs (qmv_quad.cuh)
     ("quad.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}", "-mllvm",
                   "-amdgpu-mfma-vgpr-form"])

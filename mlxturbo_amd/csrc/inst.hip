@@ -28,7 +28,6 @@ namespace mq {
 #define MQ_INST(GS)                                                  \
   template struct DequantLaunch<MQ_INST_DT, MQ_INST_BITS, GS>;       \
   template struct SkinnyLaunch<MQ_INST_DT, MQ_INST_BITS, GS>;        \
-  template struct WideLaunch<MQ_INST_DT, MQ_INST_BITS, GS>;          \
   template struct GatherLaunch<MQ_INST_DT, MQ_INST_BITS, GS>;
 #endif
 

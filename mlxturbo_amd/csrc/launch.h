@@ -39,7 +39,8 @@ struct QuadLaunch {
                  int64_t M, int64_t N, int64_t K, hipStream_t st, int* nlaunch);
 };
 
-// quantized_matmul for M > 16 rows on the MFMA tile kernel (qmm_wide.cuh);
+// quantized_matmul for M > 16 rows on the MFMA tile kernel (dense.cuh,
+// its own translation unit dense.hip);
 // with a workspace of wide_workspace_bytes(wide_plan(...), M, N) bytes the
 // K range may be split over workgroups (float partial planes plus a reduce
 // kernel).  *nlaunch counts the kernels enqueued.
@@ -223,41 +224,57 @@ inline int device_cu_count() {
   return n;
 }
 
-// Launch plan of the wide kernel: row-tile height and K splits, the pair
-// with the fewest (rounds of one workgroup per CU; every height needs 92-147
-// KB of LDS) x (time of one tile), plus the split reduction.  Tile times at
-// K=5120, measured: 71 us (64 rows), 81 (128), 105 (192), 119 (256); a tile
-// over a K slice costs ~3 us plus its share.  A last round that fills few CUs
-// costs as much as a full one (K=5120 N=17408, 68 column tiles on 256 CUs:
-// M=256 81 us with BM 128 against 112 with 256; M=512 113 with 192 against
-// 126 with 256 and 173 with 128; M=2048 362 with 192 against 406 with 256;
-// M=8192 1332 with 256 against 1515 with 192).  Splitting K serves narrow
-// matrices, whose few column tiles leave most CUs idle (K=17408 N=5120 has
-// 20), and one-round grids of wider ones: three splits put the 68 column
-// tiles of K=5120 N=17408 on 204 of 256 CUs (M=96 / 160 / 192 / 256: 48.9 /
-// 62.1 / 65.0 / 77.2 us against 59.4 / 74.9 / 79.3 / 86.5 with one, two or
-// four; graph-timed, one box).  Partial planes are float [M, N] per split,
-// written by the tile kernel and summed in split order by a reduce kernel:
-// (8 S + 2) M N bytes at ~3.5 TB/s.
+// Launch plan of the wide kernel (dense.cuh): row-tile height and K split, the
+// pair of least cost by a model fitted to measurements at K=5120 N=17408 and
+// K=17408 N=5120, M=64..8192:
+//  * a tile takes c0 (launch, first loads, stores) plus t per 64-code step;
+//    one alone 5.4 / 7.6 / 8.8 / 11.6 us plus 0.57 / 0.64 / 0.76 / 0.97 us
+//    (BM = 64 .. 256), with every CU busy the t below (M=1024, K=5120:
+//    192-row tiles 91 us a round, 256-row ones 106, 128-row ones 67);
+//  * a round of one tile per CU costs the same however few CUs it fills, but
+//    over many rounds power holds the clock, and idle CUs leave it to the
+//    others: then tiles / CUs rounds at tp per step count (K=5120: M=8192
+//    1128 us in 8.5 rounds of 256-row tiles, 1187 in 11.4 of 192-row ones;
+//    M=2048 347 in 2.1 and 302 in 2.9);
+//  * K splits sum into float [M, N] planes that a second kernel adds, 3 us
+//    plus (8 S + 2) M N bytes written and read at ~7 TB/s (they stay in the
+//    last-level cache): M=128 K=5120 39.9 us with 3 splits of 128-row tiles
+//    against 58.9 with one; M=256 K=17408 63.5 with 8 of 256-row tiles.
+// Scales are loaded for 4, 2 or 1 steps at a time (wide_unit), which K and
+// their address must allow; 256-row tiles exist for 4 and 128-row ones for 4
+// and 2 (the shorter loads' kernels of these heights do not fit the registers
+// or gain nothing).
 struct WidePlan {
   int bm = 256, splits = 1;
   double cost_us = 0.0;
 };
 
-inline WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int cus, int max_splits = 8) {
+inline int wide_unit(int64_t K, const void* s = nullptr, const void* b = nullptr) {
+  if (((uintptr_t)s | (uintptr_t)b) % 4) return 1;
+  return K % 256 == 0 ? 4 : K % 128 == 0 ? 2 : 1;
+}
+
+inline WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int cus, int max_splits = 16) {
   const int64_t cols = (N + 255) / 256;
-  const int64_t nk = K / 64;
+  const int unit = wide_unit(K);
+  const int64_t nu = K / (64 * unit);
   const int bms[4] = {64, 128, 192, 256};
-  const double tile_us[4] = {71.0, 81.0, 105.0, 119.0};   // one tile at K=5120, measured
+  const double c0[4] = {5.4, 7.6, 8.8, 11.6};
+  const double t[4] = {0.59, 0.72, 1.06, 1.24};
+  const double tp[4] = {0.62, 0.83, 1.18, 1.48};
   WidePlan best;
   bool first = true;
-  for (int sp = 1; sp <= max_splits; sp = sp == 2 ? 3 : sp == 3 ? 4 : 2 * sp) {   // 1 2 3 4 8
-    if (sp > 1 && nk / sp < 8) break;                 // at least 8 k-steps per split
+  for (int sp = 1; sp <= max_splits; ++sp) {
+    const double steps = (double)(unit * ((nu + sp - 1) / sp));
+    if (sp > 1 && steps < 8) break;             // at least 8 k-steps per split
     for (int i = 3; i >= 0; --i) {
-      const int64_t wgs = cols * ((M + bms[i] - 1) / bms[i]) * sp;
-      const double tile = (sp > 1 ? 3.0 : 0.0) + tile_us[i] * ((double)K / sp) / 5120.0;
-      double cost = (double)((wgs + cus - 1) / cus) * tile;
-      if (sp > 1) cost += (8.0 * sp + 2.0) * (double)M * (double)N / 3.5e6;
+      if ((bms[i] == 256 && unit < 4) || (bms[i] == 128 && unit < 2)) continue;
+      const int64_t tiles = cols * ((M + bms[i] - 1) / bms[i]) * sp;
+      const double rounds = (double)((tiles + cus - 1) / cus);
+      double cost = rounds * (c0[i] + t[i] * steps);
+      const double held = (double)tiles / cus * (tp[i] * steps) + c0[i];
+      if (held > cost) cost = held;
+      if (sp > 1) cost += 3.0 + (8.0 * sp + 2.0) * (double)M * (double)N / 7.0e6;
       if (first || cost < best.cost_us) {
         best.bm = bms[i];
         best.splits = sp;
@@ -280,18 +297,6 @@ inline bool wide_eligible(int64_t M, int64_t N, int64_t K, int bits, int gs) {
   return M > 16 && K % 64 == 0 && (bits == 4 || bits == 8) && gs >= 32 && gs % 32 == 0;
 }
 
-// Wide tile or 16-row skinny launches for M > 16 rows: the cheaper by a
-// model fitted to measurements.  Few column tiles starve the wide grid
-// (K=17408 N=5120: 20 tiles; M=17..64 took 229-249 us wide against 40-87
-// in 16-row launches; K=4096 N=4096: 48 against 12-29), while at K=5120
-// N=17408 the wide tile wins from M ~ 70.  Skinny launch time: about 3 us
-// plus the weight bytes at 3.6 TB/s for one row, x1.15 for 2-4 rows, x1.4
-// for 5-8, x1.65 for 9-16; on matrices of 640+ row tiles and 48+ rows per CU
-// (the shared-x workgroups of 5-16 rows) x1.35 for 5-8 and x1.42 for 9-16
-// (K=5120 N=17408: 20.7 and 21.8 us against 15.4 for the one-row model), and
-// 17-32 rows there in one launch at x1.5 (two 16-row A tiles per weight
-// fragment: M=17/24/32 22.0/21.6/21.1 us, one process).
-// split_ok: a workspace is available for K splits.
 // Rows per launch of the shared-x skinny workgroups on this matrix (the
 // launch conditions of qmv.cuh restated for the route model): 32 when a
 // launch of two 16-row A tiles fits, 16 when only the 5-16-row launch does,
@@ -351,18 +356,27 @@ inline size_t skinny_split_bytes(int64_t M, int64_t N, int64_t K, int bits, int 
   return (size_t)most * N * 8 * sizeof(float);
 }
 
+// Wide tile or skinny launches for M > 16 rows.  Up to 64 rows stay on the
+// skinny family wherever it takes them in launches of 32 (shared x) or 64
+// rows (split K slices): there every 16 rows have the bits of their own
+// 16-row call, which verify widths rely on.  Elsewhere the cheaper by a model
+// fitted to measurements: skinny launches take about 3 us plus the weight
+// bytes at 3.6 TB/s for one row, x1.15 for 2-4 rows, x1.4 for 5-8, x1.65 for
+// 9-16; on matrices of 640+ row tiles and 48+ rows per CU (the shared-x
+// workgroups of 5-16 rows) x1.35 for 5-8 and x1.42 for 9-16 (K=5120 N=17408:
+// 20.7 and 21.8 us against 15.4 for the one-row model), and 17-32 rows there
+// in one launch at x1.5 (two 16-row A tiles per weight fragment: M=17/24/32
+// 22.0/21.6/21.1 us, one process); the wide tile by wide_plan (K=5120 N=17408:
+// M=96 from the third row of tiles on, 40 us at 128 rows against 66 in 32-row
+// launches).  split_ok: a workspace is available for K splits.
 inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus,
                        bool split_ok) {
   if (!wide_eligible(M, N, K, bits, gs)) return false;
-  // The wide tile never streams its weights faster than ~0.9 TB/s at these
-  // widths (few bytes in flight per CU: M=32 48.9 us, M=96 53.6 at K=5120
-  // N=17408, M=64 49.8 at K=17408 N=5120), which the tile-time model, fitted
-  // on full rounds, does not see.
-  const double wbytes = (double)N * (double)K * bits / 8.0;
-  double wide_us = wide_plan(M, N, K, cus, split_ok ? 8 : 1).cost_us;
-  if (wide_us < wbytes / 0.9e6) wide_us = wbytes / 0.9e6;
-  const double one = 3.0 + wbytes / 3.6e6;
   const int sx = skinny_shared_x_rows(N, K, bits, gs, cus);
+  if (M <= 64 && (sx == 32 || (split_ok && skinny_split_slices(M, N, K, bits, gs)))) return false;
+  const double wbytes = (double)N * (double)K * bits / 8.0;
+  const double wide_us = wide_plan(M, N, K, cus, split_ok ? 16 : 1).cost_us;
+  const double one = 3.0 + wbytes / 3.6e6;
   const bool shared_x = sx > 0;
   double skinny_us = 0.0;
   for (int64_t m0 = 0, step = 16; m0 < M; m0 += step) {

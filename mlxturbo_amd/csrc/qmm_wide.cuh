@@ -1,15 +1,9 @@
-// Wide (prefill) quantized matmul: out[M,N] = x[M,K] . deq(W[N,K])^T for M > 16,
-// and the same tile over expert-grouped rows for prefill gather_qmm.
+// Expert-grouped tiles of prefill gather_qmm with dequantized weights in LDS.
 //
-// Reference behaviour: mlxturbo/kernels/qmm_wide.py:456-502 (MLX steel
-// qmm_t with a 64-row tile), reached from fused._qmm_wide_dispatch
-// (fused.py:3477-3499) for prefill chunks; the MLX loader dequantizes each W
-// tile to T in threadgroup memory (_steel_flat.py:1324-1335).  The grouped
-// form follows moe_grouped_gemm.qmm_segmented (moe_grouped_gemm.py:913-1066):
-// rows sorted by expert, each tile belongs to one expert.
+// Reference behaviour: moe_grouped_gemm.qmm_segmented (moe_grouped_gemm.py:
+// 913-1066): rows sorted by expert, each tile belongs to one expert.
 //
-// CDNA4 design (compute-bound: arithmetic intensity 1247-3483 FLOP/B at
-// M = 512..8192, above the ~312 FLOP/B ridge):
+// CDNA4 design:
 //  * Block tile BM x 256, BK = 64 codes, 512 threads = 8 waves, two per SIMD
 //    (one wave per SIMD left the LDS reads latency-bound: measured 213 B/ns
 //    per CU with one wave per SIMD against 430 with four).  BM = 256: waves
@@ -24,52 +18,23 @@
 //    other buffer; the loop body is straight-line so the compiler can
 //    interleave the stores with the MFMAs.  With one register stage, 44% of
 //    wave cycles waited on global loads (SQ_WAIT_INST_ANY).
-//  * x, W, scales and biases are read with buffer loads; rows past M (or past
-//    N) are past the buffer range and read zeros, so no row clamping.
+//  * x, W, scales and biases are read with buffer loads; rows past the
+//    segment (or past N) are past the buffer range and read zeros.
 //  * Each weight is dequantized once per BM output rows; a whole tile whose
 //    scales include |s| >= 2^100 (never in real checkpoints) is recomputed on
 //    the plain float dequantization route: the fast route checks each scale
 //    as it uses it, so no tile waits for a scan of its scales before its
 //    first weight load.
 #pragma once
-#include <type_traits>
-
-#include "launch.h"
+#include "stream_tile.cuh"
 
 namespace mq {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWideBN = 256, kWideBK = 64, kWideNT = 512;
 constexpr int kWideLD = kWideBK + 8;  // LDS row stride in 16-bit elements (144 bytes)
 
 template <int BM>
 constexpr size_t wide_lds_bytes() { return 2 * (size_t)(BM + kWideBN) * kWideLD * 2; }
-
-template <int DT>
-__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-  if constexpr (DT == kBF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0,
-                                                   0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(bitcast<f16x8>(a), bitcast<f16x8>(b), c, 0, 0,
-                                                  0);
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t wide_rsrc(const void* base, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0,
-                                           (int)(bytes < 0x7fffffff ? bytes : 0x7fffffff),
-                                           0x00020000);
-}
-
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 // One BM x 256 output tile over k-steps kt0 .. kt0 + nkl - 1 (64 codes each).
 // x rows come from xrsrc at per-row byte offsets xrow_off(r) (past the range
@@ -342,67 +307,6 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
     }
 }
 
-// Dense rows: grid (ceil(N / 256), ceil(M / BM), splits), 512 threads,
-// dynamic LDS wide_lds_bytes<BM>(); 256 * K * 2 < 2^31 and 256 * K * BITS / 8
-// < 2^31.  With part == nullptr (splits == 1) the tile rounds its sums into
-// out; otherwise split z sums k-steps [z nk / splits, (z + 1) nk / splits)
-// into the float plane part[z] ([M, N]) and wide_reduce_kernel adds the
-// planes in split order.
-template <int DT, int BITS, int GS, int BM>
-__global__ __launch_bounds__(kWideNT) void qmm_wide_kernel(const uint16_t* __restrict__ x,
-                                                           const uint32_t* __restrict__ w,
-                                                           const uint16_t* __restrict__ scales,
-                                                           const uint16_t* __restrict__ biases,
-                                                           uint16_t* __restrict__ out,
-                                                           float* __restrict__ part, int M,
-                                                           int N, int K) {
-  extern __shared__ __align__(16) uint16_t wide_smem[];
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * kWideBN;
-  const int mrows = min(BM, M - m0);
-  const int64_t G = K / GS;
-  const int nk = K / kWideBK, z = blockIdx.z, splits = gridDim.z;
-  const int kt0 = (int)((int64_t)nk * z / splits), kt1 = (int)((int64_t)nk * (z + 1) / splits);
-  // descriptors cover this tile's rows only: rows past M read zeros, no
-  // 64-bit offsets inside the tile
-  const auto xr = wide_rsrc(x + (int64_t)m0 * K, (int64_t)mrows * K * 2);
-  auto xrow_off = [&](int r) { return (uint32_t)r * (uint32_t)K * 2u; };
-  if (part) {
-    float* pt = part + ((int64_t)z * M + m0) * N + n0;
-    auto store = [&](int r, int c, float v) {
-      if (r < mrows) pt[(int64_t)r * N + c] = v;
-    };
-    wide_tile<DT, BITS, GS, BM>(xr, xrow_off, w + (int64_t)n0 * K * BITS / 32, scales + n0 * G,
-                                biases + n0 * G, min(kWideBN, N - n0), K, kt0, kt1 - kt0, store,
-                                wide_smem);
-  } else {
-    uint16_t* ot = out + (int64_t)m0 * N + n0;
-    auto store = [&](int r, int c, float v) {
-      if (r < mrows) ot[(int64_t)r * N + c] = T16<DT>::round1(v);
-    };
-    wide_tile<DT, BITS, GS, BM>(xr, xrow_off, w + (int64_t)n0 * K * BITS / 32, scales + n0 * G,
-                                biases + n0 * G, min(kWideBN, N - n0), K, kt0, kt1 - kt0, store,
-                                wide_smem);
-  }
-}
-
-// out = round(sum over splits of part[s]) in split order, 4 elements per
-// thread; grid ceil(M * N / 1024), 256 threads.
-template <int DT>
-__global__ __launch_bounds__(256) void wide_reduce_kernel(const float* __restrict__ part,
-                                                          uint16_t* __restrict__ out,
-                                                          int64_t MN, int splits) {
-  const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int64_t i = i0 + e;
-    if (i < MN) {
-      float v = part[i];
-      for (int z = 1; z < splits; ++z) v += part[(int64_t)z * MN + i];
-      out[i] = T16<DT>::round1(v);
-    }
-  }
-}
-
 // One expert-grouped tile (prefill gather_qmm, reference moe_grouped_gemm.py:
 // 913-1066): segment seg of the prep tables in ws (up to BM / Mi pairs of one
 // expert, pairs sorted by expert) times the 256 columns from n0.  Pair p
@@ -513,50 +417,6 @@ __global__ __launch_bounds__(kWideNT) void qmm_grouped_classes_kernel(
   else
     grouped_body<DT, BITS, GS, 64>(x, w, scales, biases, lhs, out, ws, P, B, Mi, N, K, E, seg,
                                    col * kWideBN, wide_smem, s_xoff, s_orow);
-}
-
-template <int DT, int BITS, int GS, int BM>
-inline int wide_launch_bm(const void* x, const uint32_t* w, const void* s, const void* b,
-                          void* out, int64_t M, int64_t N, int64_t K, int splits, void* ws,
-                          hipStream_t st) {
-  static std::atomic<uint64_t> lds_set{0};
-  if (hipError_t e = ensure_lds_limit(
-          reinterpret_cast<const void*>(&qmm_wide_kernel<DT, BITS, GS, BM>),
-          (int)wide_lds_bytes<BM>(), lds_set))
-    return (int)e;
-  float* part = splits > 1 ? static_cast<float*>(ws) : nullptr;
-  const dim3 grid((unsigned)((N + kWideBN - 1) / kWideBN), (unsigned)((M + BM - 1) / BM),
-                  (unsigned)splits);
-  hipLaunchKernelGGL((qmm_wide_kernel<DT, BITS, GS, BM>), grid, dim3(kWideNT),
-                     wide_lds_bytes<BM>(), st, (const uint16_t*)x, w, (const uint16_t*)s,
-                     (const uint16_t*)b, (uint16_t*)out, part, (int)M, (int)N, (int)K);
-  if (splits > 1) {
-    const int64_t MN = M * N;
-    hipLaunchKernelGGL((wide_reduce_kernel<DT>), dim3((unsigned)((MN + 1023) / 1024)), dim3(256),
-                       0, st, (const float*)part, (uint16_t*)out, MN, splits);
-  }
-  return 0;
-}
-
-template <int DT, int BITS, int GS>
-int WideLaunch<DT, BITS, GS>::run(const void* x, const uint32_t* w, const void* s, const void* b,
-                                  void* out, int64_t M, int64_t N, int64_t K, void* ws,
-                                  size_t ws_bytes, hipStream_t st, int* nlaunch) {
-  // one tile's x rows and weight rows must fit a 31-bit buffer range
-  if (K * 2 * 256 >= ((int64_t)1 << 31) || M > ((int64_t)1 << 31) / 256 * 256)
-    return kStatusUnsupported;
-  const int cus = device_cu_count();
-  WidePlan plan = wide_plan(M, N, K, cus);
-  if (plan.splits > 1 && (!ws || ws_bytes < wide_workspace_bytes(plan, M, N)))
-    plan = wide_plan(M, N, K, cus, 1);
-  const int splits = plan.splits;
-  *nlaunch += splits > 1 ? 2 : 1;
-  switch (plan.bm) {
-    case 64: return wide_launch_bm<DT, BITS, GS, 64>(x, w, s, b, out, M, N, K, splits, ws, st);
-    case 128: return wide_launch_bm<DT, BITS, GS, 128>(x, w, s, b, out, M, N, K, splits, ws, st);
-    case 192: return wide_launch_bm<DT, BITS, GS, 192>(x, w, s, b, out, M, N, K, splits, ws, st);
-    default: return wide_launch_bm<DT, BITS, GS, 256>(x, w, s, b, out, M, N, K, splits, ws, st);
-  }
 }
 
 }  // namespace mq
