@@ -511,15 +511,6 @@ inline int launch_grouped_class(const void* x, const uint32_t* w, const void* s,
   return 0;
 }
 
-// Segments of the pairs of a size class when experts with at least C pairs
-// are cut into segments of R pairs: at most P / R + P / C (one partial
-// segment per expert of the class) and never more than P.
-inline int64_t class_seg_bound(int64_t P, int64_t R, int64_t C, int64_t E) {
-  int64_t b = (P + R - 1) / R + (C > 0 ? P / C : E + 1);
-  if (b > E + 1 + (P + R - 1) / R) b = E + 1 + (P + R - 1) / R;
-  return b < P ? b : P;
-}
-
 // Prefill gather_qmm: prep tables, then the expert-grouped MFMA tile kernel.
 // One row-tile height for every expert (BM rows) when the expected rows per
 // expert call for it, or size classes: experts with 192+ rows get 256-row
@@ -562,54 +553,33 @@ inline int launch_grouped_bm(const void* x, const uint32_t* w, const void* s, co
   return 0;
 }
 
-// The thin grouped kernel (grouped.cuh) over two-class tables already built
-// in ws (launch_thin_tables: segments of R = 64 / M pairs, and of 2 R for
-// experts with more than R pairs).  GLU: gate bank (w, s, b) and up bank
-// (w2, s2, b2), out = SwiGLU of the two gathers (N columns).
+// The thin grouped kernels over two-class tables already built in ws
+// (launch_thin_tables: segments of R = 64 / M pairs, and of 2 R for experts
+// with more than R pairs, which run as two 64-row tiles: 128-row tiles of 4
+// waves took 261 us against 176 on the K=512 down bank).  GLU: gate bank (w,
+// s, b) and up bank (w2, s2, b2), out = SwiGLU of the two gathers (N columns).
+// 4-bit banks stream through LDS (grouped.cuh), 8-bit banks through registers
+// (grouped8.cuh); each file states the other's time on its banks.
 template <int DT, int BITS, int GS, bool GLU>
 inline int launch_thin_kernel(const void* x, const uint32_t* w, const void* s, const void* b,
                               const uint32_t* w2, const void* s2, const void* b2,
                               const int32_t* lhs, void* out, int64_t P, int64_t B, int64_t M,
                               int64_t N, int64_t K, int64_t E, const void* ws, hipStream_t st) {
-  const int R = (int)(kThinBM / M);
-  // 4 waves (256 columns) per workgroup for 4-bit weights and at short K, 8
-  // (512 columns, so each x tile serves twice the columns) for 8-bit weights
-  // above K = 1024.  Config-4 banks, 2048 tokens x top-8, one process: down
-  // (K=512) 143 / 122 us zipf / uniform with 4 against 173 / 141 with 8.
-  // Gate/up (K=2048): 4-bit 4-wave tiles stream their weights through LDS
-  // (the DMA form in grouped.cuh) and take 275 / 241 us against 285 / 261
-  // with 8 waves; the fused SwiGLU layer 425 against 447 us zipf.  Without
-  // that stream (8-bit) 8 waves won: 279 / 222 against 302 / 253 for the
-  // size-class wide tiles and 282 / 264 with 16 waves (whose 128-register
-  // budget spills).
-  const int nwv = (K <= 1024 || BITS == 4) ? 4 : 8;
-  const int64_t bn = (GLU ? 32 : 64) * nwv;     // output columns per tile
-  const int64_t ncol = (N + bn - 1) / bn;
-  // 8 waves: experts with more than 64 rows take 128-row tiles, which read
-  // their weights once per 128 rows (the workgroup's register budget
-  // already holds one workgroup per CU, so the taller tile costs no
-  // occupancy).  4 waves run those segments as two 64-row tiles (128-row
-  // tiles with 4 waves: config-4 down 261 against 176 us zipf), the same
-  // work as one-class tables, so one table build serves both widths.
-  const int64_t h1 = nwv == 4 ? 2 : 1;
-  int64_t nwg = 0;
-  for (const int64_t sb : {h1 * class_seg_bound(P, 2 * R, R + 1, E), class_seg_bound(P, R, 0, E)})
-    nwg += (sb * ncol + 7) / 8 * 8;
-  if (nwg > INT32_MAX) return kStatusUnsupported;
-  const dim3 grid((unsigned)nwg);
-#define MQ_THIN(NWV, HALVES)                                                                    \
-  hipLaunchKernelGGL((qmm_grouped_thin_kernel<DT, BITS, GS, 2, NWV, true, HALVES, GLU>), grid,  \
-                     dim3(64 * NWV), 0, st, (const uint16_t*)x, w, (const uint16_t*)s,           \
-                     (const uint16_t*)b, w2, (const uint16_t*)s2, (const uint16_t*)b2, lhs,      \
-                     (uint16_t*)out, (const int32_t*)ws, (int)P, (int)B, (int)M, (int)N, (int)K, \
-                     (int)E, 0)
-  if (nwv == 4) MQ_THIN(4, true);
-  else MQ_THIN(8, false);
-#undef MQ_THIN
-  return 0;
+  if constexpr (BITS == 8) {
+    return Thin8Launch<DT, GS, GLU>::run(x, w, s, b, w2, s2, b2, lhs, out, P, B, M, N, K, E, ws,
+                                         st);
+  } else {
+    const int64_t nwg = thin_grid(P, M, N, E, GLU);
+    if (nwg > INT32_MAX) return kStatusUnsupported;
+    hipLaunchKernelGGL((qmm_grouped_thin_kernel<DT, GS, GLU>), dim3((unsigned)nwg), dim3(256), 0,
+                       st, (const uint16_t*)x, w, (const uint16_t*)s, (const uint16_t*)b, w2,
+                       (const uint16_t*)s2, (const uint16_t*)b2, lhs, (uint16_t*)out,
+                       (const int32_t*)ws, (int)P, (int)B, (int)M, (int)N, (int)K, (int)E);
+    return 0;
+  }
 }
 
-// Prefill gather_qmm with thin experts: the register-B grouped kernel over
+// Prefill gather_qmm with thin experts: a thin grouped kernel over
 // two-class tables, built here unless the caller built them for this
 // routing already (prepped).
 template <int DT, int BITS, int GS>

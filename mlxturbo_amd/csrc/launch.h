@@ -113,6 +113,17 @@ struct SwigluTablesLaunch {
                  const void* tables, hipStream_t st, int* nlaunch);
 };
 
+// The thin grouped kernel of 8-bit banks (grouped8.cuh, instantiated in
+// dense.hip) over tables that launch_thin_tables built in ws; GLU: gate bank (w, s, b) and
+// up bank (w2, s2, b2), out = SwiGLU of the two gathers.
+template <int DT, int GS, bool GLU>
+struct Thin8Launch {
+  static int run(const void* x, const uint32_t* w, const void* s, const void* b,
+                 const uint32_t* w2, const void* s2, const void* b2, const int32_t* lhs,
+                 void* out, int64_t P, int64_t B, int64_t M, int64_t N, int64_t K, int64_t E,
+                 const void* ws, hipStream_t st);
+};
+
 // Down projection with the MoE combine folded in (gather.cuh), decode widths:
 // x [T * top_k, K] (one row per pair), rhs and cw (float router weights)
 // [T * top_k], out [T, N] = the combine of mq_moe_combine (inv = NULL) over
@@ -442,7 +453,20 @@ constexpr int kPrepLaunches = 2;
 int launch_prep(const int32_t* rhs, const int32_t* lhs, int64_t P, int64_t E, int64_t B, int R,
                 void* ws, hipStream_t st, int R1 = 0, int C1 = 0, int R2 = 0, int C2 = 0);
 
-// Whether gather_qmm runs the thin grouped kernel (grouped.cuh): prefill
+// Segments of the pairs of a size class when experts with at least C pairs
+// are cut into segments of R pairs: at most P / R + P / C (one partial
+// segment per expert of the class) and never more than P.
+inline int64_t class_seg_bound(int64_t P, int64_t R, int64_t C, int64_t E) {
+  int64_t b = (P + R - 1) / R + (C > 0 ? P / C : E + 1);
+  if (b > E + 1 + (P + R - 1) / R) b = E + 1 + (P + R - 1) / R;
+  return b < P ? b : P;
+}
+
+// Rows of the thin grouped kernels' tiles.
+constexpr int kThinBM = 64;
+
+// Whether gather_qmm runs a thin grouped kernel (grouped.cuh; 8-bit
+// banks grouped8.cuh): prefill
 // widths (P M >= kGroupedMinRows output rows), banks within the prep
 // tables, fewer than 96 rows per active expert, K <= 2048 in whole 64-code
 // steps.  The same routing then serves calls of different K (a MoE layer's
@@ -453,7 +477,16 @@ inline bool gather_thin_path(int64_t P, int64_t M, int64_t K, int64_t E) {
   return P * M / (active > 0 ? active : 1) < 96;
 }
 
-// The thin kernel's tables (launch_prep): segments of R = 64 / M pairs, and
+// Workgroups of a thin grouped kernel: its segments' bound (two tiles for the
+// long ones) x column tiles of 256 weight rows, each class in whole eights.
+inline int64_t thin_grid(int64_t P, int64_t M, int64_t N, int64_t E, bool glu) {
+  const int64_t R = kThinBM / M, bn = glu ? 128 : 256, ncol = (N + bn - 1) / bn;
+  const int64_t n1 = 2 * class_seg_bound(P, 2 * R, R + 1, E) * ncol;
+  const int64_t n0 = class_seg_bound(P, R, 0, E) * ncol;
+  return (n1 + 7) / 8 * 8 + (n0 + 7) / 8 * 8;
+}
+
+// The thin kernels' tables (launch_prep): segments of R = 64 / M pairs, and
 // of 2 R pairs for experts with more than R pairs (class 1).
 inline int launch_thin_tables(const int32_t* rhs, const int32_t* lhs, int64_t P, int64_t E,
                               int64_t B, int64_t M, void* ws, hipStream_t st) {

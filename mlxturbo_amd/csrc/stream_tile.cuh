@@ -172,11 +172,6 @@ __device__ __forceinline__ void stream_tile(
     rb[j] = wide_rsrc(up ? biases2 : biases, (int64_t)ncols * G * 2);
   }
   uint32_t dmo[DM];
-#pragma unroll
-  for (int i = 0; i < DM; ++i) {
-    const int r = 8 * (wave * DM + i) + (lane >> 3);
-    dmo[i] = xrow_off(r) + 16u * (uint32_t)((lane & 7) ^ row_swz(r));
-  }
   uint32_t wo[2], so[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -329,9 +324,18 @@ __device__ __forceinline__ void stream_tile(
   static_for<0, RU>([&](auto rc) {
     static_for<0, 4>([&](auto ic) { sload(U * decltype(rc)::value, rc, ic); });
   });
-  static_for<0, NL>([&](auto vc) { load(0, I0{}, vc); });
-  static_for<0, NL>([&](auto vc) { load(1, I1{}, vc); });
-  static_for<0, NL>([&](auto vc) { load(2, I2{}, vc); });
+  // the weights first: x rows may have to be looked up (xrow_off)
+  static_for<DM, NL>([&](auto vc) { load(0, I0{}, vc); });
+  static_for<DM, NL>([&](auto vc) { load(1, I1{}, vc); });
+  static_for<DM, NL>([&](auto vc) { load(2, I2{}, vc); });
+#pragma unroll
+  for (int i = 0; i < DM; ++i) {
+    const int r = 8 * (wave * DM + i) + (lane >> 3);
+    dmo[i] = xrow_off(r) + 16u * (uint32_t)((lane & 7) ^ row_swz(r));
+  }
+  static_for<0, DM>([&](auto vc) { load(0, I0{}, vc); });
+  static_for<0, DM>([&](auto vc) { load(1, I1{}, vc); });
+  static_for<0, DM>([&](auto vc) { load(2, I2{}, vc); });
   // the x loads alone are counted here: the others may move below the barrier
   barrier(std::integral_constant<int, 2 * DM>{});
   group(I0{}, I0{});
