@@ -16,11 +16,11 @@
 //   scale = q0 != 0 ? edge / q0 : scale0; bias = q0 == 0 ? 0 : edge;
 //   code = clamp(rint((w - bias) / scale), 0, 2^bits - 1), NaN -> 0.
 // Every operation is one correctly rounded IEEE float32 operation (the
-// division is hipcc's correctly rounded sequence, rint is v_rndne), so the
-// result is a deterministic function of the input bits.  NaN propagates
-// through the group minimum and maximum.  The group's lanes (group_size / 8
-// consecutive lanes of a wave) combine their minima and maxima with
-// cross-lane exchanges.
+// division is hipcc's correctly rounded sequence or an equal one, rint is
+// v_rndne), so the result is a deterministic function of the input bits.  NaN
+// propagates through the group minimum and maximum.  The group's lanes
+// (group_size / 16 consecutive lanes of a wave) combine their minima and
+// maxima with cross-lane exchanges.
 #include "launch.h"
 
 namespace mq {
@@ -101,37 +101,114 @@ __device__ __forceinline__ uint64_t load_octet_codes(const uint8_t* wq, int64_t 
   }
 }
 
-// One thread per octet of codes; group_size / 8 consecutive lanes form a
-// group.  The loop bound is uniform per wave (octets is a multiple of the
-// group's lane count and every wave starts on a multiple of 64), so every
-// lane of a group takes part in the exchanges.
+// v of the lane's partner in an exchange over 2 OFF lanes that are equal in
+// halves of OFF already (quad_perm, then the half-row and row mirrors: VALU
+// moves, no trip through LDS).
+template <int OFF>
+__device__ __forceinline__ float exchange(float v) {
+  static_assert(OFF == 1 || OFF == 2 || OFF == 4, "exchanges within 8 lanes");
+  constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : 0x141;
+  return __uint_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_uint(v), ctrl, 0xF, 0xF, true));
+}
+
+// f(1), f(2), .. below L
+template <int L, int OFF = 1, class F>
+__device__ __forceinline__ void for_offsets(F f) {
+  if constexpr (OFF < L) {
+    f(std::integral_constant<int, OFF>{});
+    for_offsets<L, 2 * OFF>(f);
+  }
+}
+
+// Codes of two octets, lowest code lowest in p[0], then p[1].
+// RECIP: (v - bias) / scale by a reciprocal r = RN(1 / scale).  q0 = RN(a r) is
+// within two units in the last place of a / scale, q1 = q0 + r (a - q0 scale)
+// is therefore one of the two floats next to it, and then q2 = q1 + r (a - q1
+// scale) is a / scale correctly rounded (Markstein, IBM J. Res. Dev. 34, 1990),
+// its remainder being exact by fma.  Requires finite a and a |scale| in
+// [2^-26, 2^100]: r is normal and nothing that decides a code underflows.
+template <int BITS, bool RECIP>
+__device__ __forceinline__ void codes16(const float v[16], float scale, float bias,
+                                        uint64_t p[2]) {
+  const float nb = (float)((1 << BITS) - 1);
+  const float r = RECIP ? 1.0f / scale : 0.f;
+  p[0] = p[1] = 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float a = v[j] - bias;
+    float q;
+    if constexpr (RECIP) {
+      q = a * r;
+      q = __builtin_fmaf(__builtin_fmaf(-q, scale, a), r, q);
+      q = __builtin_fmaf(__builtin_fmaf(-q, scale, a), r, q);
+      q = __builtin_amdgcn_fmed3f(__builtin_rintf(q), 0.f, nb);
+    } else {
+      q = __builtin_rintf(a / scale);
+      q = (q != q) ? 0.f : __builtin_fminf(__builtin_fmaxf(q, 0.f), nb);
+    }
+    p[j / 8] |= (uint64_t)(uint32_t)q << (BITS * (j % 8));
+  }
+}
+
+// One thread per two octets of codes; group_size / 16 consecutive lanes form a
+// group.  The loop bound is uniform per wave (the octets are a multiple of the
+// group's and every wave starts on a multiple of 128), so every lane of a group
+// takes part in the exchanges.
+//
+// A correctly rounded division per code and NaN-keeping minima are VALU work: one
+// octet per thread took 72.9 us for 89 M codes, bfloat16 -> 4 bits, groups of 64
+// (3.1 TB/s; 24 us less so, which is about what its bytes take).  So a wave whose inputs are finite and whose
+// scales are of ordinary size takes plain minima (v_med3 with an infinity)
+// and divides by a reciprocal; two octets per thread share the four divisions
+// of a group's scale.  Any other wave runs every operation as written above.
 template <int DT, int BITS, int GS>
 __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ w,
                                                        uint8_t* __restrict__ wq,
                                                        void* __restrict__ scales,
                                                        void* __restrict__ biases, int64_t octets) {
-  constexpr int L = GS / 8;
-  const float nb = (float)((1 << BITS) - 1);
+  constexpr int L = GS / 16;
+  const float nb = (float)((1 << BITS) - 1), inf = __builtin_inff();
   const int lane = threadIdx.x & 63;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63); base < octets;
+  const int64_t stride = 2 * (int64_t)gridDim.x * blockDim.x;
+  for (int64_t base = 2 * ((int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63)); base < octets;
        base += stride) {
-    const int64_t o = base + lane;
+    const int64_t o = base + 2 * lane;          // octets is even
     const bool live = o < octets;
-    float v[8];
+    float v[16];
     if (live) {
       load_octet<DT>(w, o, v);
+      load_octet<DT>(w, o + 1, v + 8);
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = 0.f;
+      for (int j = 0; j < 16; ++j) v[j] = 0.f;
     }
+    // NaN where an input is infinite or NaN (or a sum overflows: also taken
+    // the long way)
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sum += v[j];
+    const bool finite = __builtin_fabsf(sum) < inf;
     float hi = v[0], lo = v[0];
+    if (__all(finite)) {
 #pragma unroll
-    for (int j = 1; j < 8; ++j) { hi = nan_max(hi, v[j]); lo = nan_min(lo, v[j]); }
+      for (int j = 1; j < 16; ++j) {
+        hi = __builtin_amdgcn_fmed3f(hi, v[j], inf);
+        lo = __builtin_amdgcn_fmed3f(lo, v[j], -inf);
+      }
+      for_offsets<L>([&](auto oc) {
+        constexpr int OFF = decltype(oc)::value;
+        hi = __builtin_amdgcn_fmed3f(hi, exchange<OFF>(hi), inf);
+        lo = __builtin_amdgcn_fmed3f(lo, exchange<OFF>(lo), -inf);
+      });
+    } else {
 #pragma unroll
-    for (int off = 1; off < L; off <<= 1) {
-      hi = nan_max(hi, __shfl_xor(hi, off));
-      lo = nan_min(lo, __shfl_xor(lo, off));
+      for (int j = 1; j < 16; ++j) { hi = nan_max(hi, v[j]); lo = nan_min(lo, v[j]); }
+      for_offsets<L>([&](auto oc) {
+        constexpr int OFF = decltype(oc)::value;
+        hi = nan_max(hi, __shfl_xor(hi, OFF));   // of several NaNs the first
+        lo = nan_min(lo, __shfl_xor(lo, OFF));
+      });
     }
     const float d = (hi - lo) / nb;
     float scale = (d != d) ? d : (d > 1e-7f ? d : 1e-7f);
@@ -141,18 +218,18 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
     const float q0 = __builtin_rintf(edge / scale);
     if (q0 != 0.0f) scale = edge / q0;
     const float bias = (q0 == 0.0f) ? 0.0f : edge;
-    uint64_t packed = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float q = __builtin_rintf((v[j] - bias) / scale);
-      q = (q != q) ? 0.f : __builtin_fminf(__builtin_fmaxf(q, 0.f), nb);
-      packed |= (uint64_t)(uint32_t)q << (BITS * j);
-    }
+    uint64_t packed[2];
+    const float as = __builtin_fabsf(scale);
+    if (__all(finite && as >= 0x1p-26f && as <= 0x1p100f))
+      codes16<BITS, true>(v, scale, bias, packed);
+    else
+      codes16<BITS, false>(v, scale, bias, packed);
     if (live) {
-      store_octet<BITS>(wq, o, packed);
+      store_octet<BITS>(wq, o, packed[0]);
+      store_octet<BITS>(wq, o + 1, packed[1]);
       if ((lane & (L - 1)) == 0) {
-        store_param<DT>(scales, o / L, scale);
-        store_param<DT>(biases, o / L, bias);
+        store_param<DT>(scales, o / (2 * L), scale);
+        store_param<DT>(biases, o / (2 * L), bias);
       }
     }
   }
@@ -228,7 +305,7 @@ int by_format(int dtype, int bits, int gs, A... args) {
 template <int DT, int BITS, int GS>
 struct QuantizeRun {
   static int run(const void* w, uint32_t* wq, void* s, void* b, int64_t octets, hipStream_t st) {
-    hipLaunchKernelGGL((quantize_kernel<DT, BITS, GS>), dim3(octet_grid(octets)), dim3(256), 0,
+    hipLaunchKernelGGL((quantize_kernel<DT, BITS, GS>), dim3(octet_grid(octets / 2)), dim3(256), 0,
                        st, w, reinterpret_cast<uint8_t*>(wq), s, b, octets);
     return 0;
   }
