@@ -64,13 +64,17 @@ class QuantizedLinear(torch.nn.Module):
         rebuilt when a tensor is replaced or written in place; ``None`` for
         configurations the full operator handles (non-affine modes, weights
         off the GPU, missing biases)."""
-        if self.mode != "affine" or self.weight.device.type != "cuda" or self.biases is None:
+        # read from the buffers once: each attribute read of a module searches
+        # its parameters first
+        bufs = self._buffers
+        w, s, b = bufs.get("weight"), bufs.get("scales"), bufs.get("biases")
+        if w is None or s is None or b is None:      # not (all) buffers any more, or no biases
+            w, s, b = self.weight, self.scales, self.biases
+        if self.mode != "affine" or not w.is_cuda or b is None:
             return None
         p = self.__dict__.get("_mq_prepared")
-        if p is None or not p.matches(self.weight, self.scales, self.biases, self.group_size,
-                                      self.bits):
-            p = ops.PreparedWeights(self.weight, self.scales, self.biases, self.group_size,
-                                    self.bits, self.mode)
+        if p is None or not p.matches(w, s, b, self.group_size, self.bits):
+            p = ops.PreparedWeights(w, s, b, self.group_size, self.bits, self.mode)
             self.__dict__["_mq_prepared"] = p
         return p
 

@@ -43,6 +43,7 @@ _DTYPE_CODE = {
 
 _GROUP_SIZES = (32, 64, 128)
 _BITS = (2, 3, 4, 5, 6, 8)
+_CODE_DTYPES = (torch.uint32, torch.int32)
 
 
 def _stream_ptr(t: torch.Tensor) -> int:
@@ -50,25 +51,29 @@ def _stream_ptr(t: torch.Tensor) -> int:
 
 
 def _require_gpu(*ts: torch.Tensor) -> torch.device:
-    dev = None
+    first = None
     for t in ts:
         if t is None:
             continue
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"expected torch.Tensor, got {type(t).__name__}")
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError(
                 "mlxturbo_amd operators run on a ROCm GPU only; got a tensor on "
                 f"{t.device} (there is no CPU fallback)")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} and {t.device}")
-    return dev
+        # by index: building and comparing torch.device objects is most of the
+        # check's time
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise ValueError(f"tensors on different devices: {first.device} and {t.device}")
+    return None if first is None else first.device
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """Row-contiguous with a 16-byte aligned base (copies only when needed)."""
+    if t.is_contiguous() and not t.data_ptr() % 16:
+        return t
     t = t.contiguous()
     if t.data_ptr() % 16:
         t = t.clone()
@@ -92,20 +97,21 @@ def _check_format(group_size: int, bits: int) -> None:
 
 def _check_quant(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                  group_size: int, bits: int) -> int:
-    if w.dtype not in (torch.uint32, torch.int32):
+    if w.dtype not in _CODE_DTYPES:
         raise ValueError(f"w must be uint32 packed codes, got {w.dtype}")
     _check_format(group_size, bits)
-    if (w.shape[-1] * 32) % bits:
-        raise ValueError(f"w last dimension {w.shape[-1]} is not whole {bits}-bit codes")
-    K = w.shape[-1] * 32 // bits
-    if scales.shape != biases.shape:
-        raise ValueError(f"scales {tuple(scales.shape)} and biases {tuple(biases.shape)} differ")
+    wshape, sshape = tuple(w.shape), tuple(scales.shape)
+    if (wshape[-1] * 32) % bits:
+        raise ValueError(f"w last dimension {wshape[-1]} is not whole {bits}-bit codes")
+    K = wshape[-1] * 32 // bits
+    if sshape != biases.shape:
+        raise ValueError(f"scales {sshape} and biases {tuple(biases.shape)} differ")
     if scales.dtype != biases.dtype:
         raise ValueError("scales and biases must have the same dtype")
-    want = (*w.shape[:-1], K // group_size)
-    if K % group_size or tuple(scales.shape) != want:
+    want = (*wshape[:-1], K // group_size)
+    if K % group_size or sshape != want:
         raise ValueError(
-            f"scales shape {tuple(scales.shape)} does not match w {tuple(w.shape)} "
+            f"scales shape {sshape} does not match w {wshape} "
             f"with group_size={group_size}, bits={bits} (expected {want})")
     return K
 
@@ -257,7 +263,8 @@ class PreparedWeights:
     key holds each tensor's version counter, so a ``copy_`` into the layer's
     weights, e.g. ``load_state_dict``, invalidates a cached aligned copy)."""
 
-    __slots__ = ("w", "s", "b", "N", "K", "group_size", "bits", "dtype", "dev", "key")
+    __slots__ = ("w", "s", "b", "N", "K", "group_size", "bits", "dtype", "dev", "index", "code",
+                 "key")
 
     def __init__(self, w, scales, biases, group_size: int = 64, bits: int = 4,
                  mode: str = "affine"):
@@ -269,6 +276,10 @@ class PreparedWeights:
         self.N = w.shape[0]
         self.w, self.s, self.b = _aligned(w), _aligned(scales), _aligned(biases)
         self.group_size, self.bits, self.dtype = group_size, bits, scales.dtype
+        self.index = w.get_device()
+        # the kernels' code of the dtype, None where they do not take the format
+        self.code = _DTYPE_CODE[self.dtype] if (
+            bits in (4, 8) and _kernel_dtype(self.dtype, self.dtype)) else None
         self.key = self._key(w, scales, biases, group_size, bits)
 
     @staticmethod
@@ -285,15 +296,16 @@ _QMM_WS_BYTES: dict = {}
 
 def quantized_matmul_prepared(x: torch.Tensor, p: PreparedWeights) -> torch.Tensor:
     """:func:`quantized_matmul` with weights validated by :class:`PreparedWeights`."""
-    if (x.device != p.dev or x.dtype != p.dtype or x.ndim < 1 or x.shape[-1] != p.K
-            or p.bits not in (4, 8) or not _kernel_dtype(x.dtype, p.dtype)):
-        return quantized_matmul(x, p.w, p.s, p.b, group_size=p.group_size, bits=p.bits)
+    shape = x.shape
     N, K = p.N, p.K
+    if (p.code is None or x.dtype != p.dtype or x.get_device() != p.index or not shape
+            or shape[-1] != K):
+        return quantized_matmul(x, p.w, p.s, p.b, group_size=p.group_size, bits=p.bits)
     M = x.numel() // K
-    out = torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=p.dev)
+    out = torch.empty((*shape[:-1], N), dtype=p.dtype, device=p.dev)
     if M == 0 or N == 0:
         return out
-    x_ = x if x.is_contiguous() and x.data_ptr() % 16 == 0 else _aligned(x)
+    x_ = _aligned(x)
     lib = _lib.lib()
     ws = None
     if M > 16:
@@ -307,10 +319,12 @@ def quantized_matmul_prepared(x: torch.Tensor, p: PreparedWeights) -> torch.Tens
         ws = _workspace(p.dev, nbytes) if nbytes else None
     rc = lib.mq_quantized_matmul_ws(x_.data_ptr(), p.w.data_ptr(), p.s.data_ptr(),
                                     p.b.data_ptr(), out.data_ptr(), M, N, K, p.group_size,
-                                    p.bits, _DTYPE_CODE[x.dtype], 1,
+                                    p.bits, p.code, 1,
                                     ws.data_ptr() if ws is not None else None,
-                                    ws.numel() if ws is not None else 0, _stream_ptr(out))
-    _lib.check(rc, "quantized_matmul")
+                                    ws.numel() if ws is not None else 0,
+                                    torch._C._cuda_getCurrentRawStream(p.index))
+    if rc:
+        _lib.check(rc, "quantized_matmul")
     return out
 
 
@@ -1001,21 +1015,26 @@ def _block_fused(x, logits, top_k, gate, up, down, sgw, shared, group_size, bits
         raise ValueError(f"shared must be ({T}, {N2}) of x's dtype")
     _require_gpu(wd, sd, bd, shared)
     dev = x.device
-    idx = torch.empty((T, top_k), dtype=torch.int32, device=dev)
-    wts = torch.empty((T, top_k), dtype=torch.float32, device=dev)
-    sgate = torch.empty((T, 1), dtype=x.dtype, device=dev) if sgw is not None else None
-    h = torch.empty((T, top_k, 1, N1), dtype=x.dtype, device=dev)
+    # one allocation for what passes between the block's stages (indices,
+    # weights, the shared gate, the hidden rows), each on 256 bytes
+    pairs = T * top_k
+    o_w = -(-4 * pairs // 256) * 256
+    o_g = 2 * o_w
+    o_h = o_g + -(-2 * T // 256) * 256
+    scratch = torch.empty(o_h + 2 * pairs * N1, dtype=torch.uint8, device=dev)
+    base = scratch.data_ptr()
     out = torch.empty((T, N2), dtype=x.dtype, device=dev)
-    x_ = _aligned(x.contiguous())
+    x_ = _aligned(x)
     lg = logits.contiguous()
     g_ = sgw.reshape(-1).contiguous() if sgw is not None else None
     sh_ = shared.contiguous() if shared is not None else None
     (wg, sg_, bg), (wu, su, bu) = gate, up
     banks = [_aligned(t) for t in (wg, sg_, bg, wu, su, bu, wd, sd, bd)]
     rc = _lib.lib().mq_moe_block(x_.data_ptr(), lg.data_ptr(), *[t.data_ptr() for t in banks],
-                                 _ptr(g_), _ptr(sh_), idx.data_ptr(), wts.data_ptr(),
-                                 _ptr(sgate), h.data_ptr(), out.data_ptr(), T, top_k, N1, K1,
-                                 N2, E, group_size, bits, _DTYPE_CODE[x.dtype], _stream_ptr(out))
+                                 _ptr(g_), _ptr(sh_), base, base + o_w,
+                                 base + o_g if g_ is not None else None, base + o_h,
+                                 out.data_ptr(), T, top_k, N1, K1, N2, E, group_size, bits,
+                                 _DTYPE_CODE[x.dtype], _stream_ptr(out))
     if rc == _EUNSUPPORTED:
         return None
     _lib.check(rc, "moe_block")
