@@ -97,6 +97,18 @@ int mq_quantize(const void* w, uint32_t* wq, void* scales, void* biases, int64_t
                 int group_size, int bits, int dtype, void* hip_stream);
 
 /*
+ * (wq, qscales, qbiases) = quantize(dequantize(w)) in one pass: mq_dequantize
+ * of (w, scales, biases) at from_group_size / from_bits followed by mq_quantize
+ * at group_size / bits, bit for bit, without the dequantized weights in memory
+ * (a layer's double quantization, mlxturbo/rebit.py:96-120).  from_bits 4 or 8,
+ * dtype bfloat16 or float16, else MQ_EUNSUPPORTED; all pointers 16-byte
+ * aligned; the outputs overlap no input.
+ */
+int mq_requantize(const uint32_t* w, const void* scales, const void* biases, int from_group_size,
+                  int from_bits, uint32_t* wq, void* qscales, void* qbiases, int64_t N, int64_t K,
+                  int group_size, int bits, int dtype, void* hip_stream);
+
+/*
  * out[M, N] = x[M, K] . dequantize(w)^T       (transpose = 1)
  * Replaces mx.quantized_matmul(x, w, scales, biases, transpose=True,
  * group_size, bits, mode="affine") as called by the reference's route layer

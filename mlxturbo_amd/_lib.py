@@ -29,6 +29,7 @@ EXPORTED = (
     "mq_set_row_identity",
     "mq_dequantize",
     "mq_quantize",
+    "mq_requantize",
     "mq_quantized_matmul",
     "mq_quantized_matmul_workspace_size",
     "mq_quantized_matmul_ws",
@@ -75,6 +76,9 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.mq_dequantize.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _int, _int, _int, _vp]
     lib.mq_quantize.restype = _int
     lib.mq_quantize.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _int, _int, _int, _vp]
+    lib.mq_requantize.restype = _int
+    lib.mq_requantize.argtypes = [_vp, _vp, _vp, _int, _int, _vp, _vp, _vp, _i64, _i64, _int,
+                                  _int, _int, _vp]
     lib.mq_quantized_matmul.restype = _int
     lib.mq_quantized_matmul.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int,
                                         _int, _int, _vp]

@@ -201,6 +201,24 @@ int mq_quantize(const void* w, uint32_t* wq, void* scales, void* biases, int64_t
   return check_launch("quantize");
 }
 
+int mq_requantize(const uint32_t* w, const void* scales, const void* biases, int from_group_size,
+                  int from_bits, uint32_t* wq, void* qscales, void* qbiases, int64_t N, int64_t K,
+                  int group_size, int bits, int dtype, void* hip_stream) {
+  int rc = check_format(w, scales, biases, N, K, from_group_size, from_bits, dtype);
+  if (!rc) rc = check_format(wq, qscales, qbiases, N, K, group_size, bits, dtype);
+  if (rc) return rc;
+  if (dtype == MQ_FLOAT32 || (from_bits != 4 && from_bits != 8))
+    return fail(MQ_EUNSUPPORTED, "requantize takes 4- and 8-bit codes of 16-bit types");
+  if (!aligned16(qscales) || !aligned16(qbiases))
+    return fail(MQ_EINVAL, "scales and biases must be 16-byte aligned");
+  if (N == 0) return MQ_OK;
+  rc = mq::launch_requantize(w, scales, biases, from_group_size, from_bits, wq, qscales, qbiases,
+                             N, K, group_size, bits, dtype,
+                             reinterpret_cast<hipStream_t>(hip_stream));
+  if (rc) return fail(rc, "requantize: no kernel for bits=%d group_size=%d", bits, group_size);
+  return check_launch("requantize");
+}
+
 size_t mq_quantized_matmul_workspace_size(int64_t M, int64_t N, int64_t K, int group_size,
                                           int bits) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size) return 0;

@@ -61,6 +61,33 @@ __device__ __forceinline__ void load_octet(const void* w, int64_t o, float v[8])
   }
 }
 
+// Octets o and o + 1 (o even) of SB-bit codes, dequantized to T (exact in
+// float: a 16-bit scale times a code is, so the fma rounds once) and back.
+template <int DT, int SB>
+__device__ __forceinline__ void load_codes16(const void* w, float s, float b, int64_t o,
+                                             float v[16]) {
+  uint32_t c[SB / 2];
+  if constexpr (SB == 8) {
+    const u32x4 t = reinterpret_cast<const u32x4*>(w)[o / 2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = t[i];
+  } else {
+    const u32x2 t = reinterpret_cast<const u32x2*>(w)[o / 2];
+    c[0] = t[0];
+    c[1] = t[1];
+  }
+  constexpr int PER = 32 / SB;
+  constexpr uint32_t MASK = (1u << SB) - 1u;
+#pragma unroll
+  for (int j = 0; j < 16; j += 2) {
+    const float q0 = (float)((c[j / PER] >> (SB * (j % PER))) & MASK);
+    const float q1 = (float)((c[j / PER] >> (SB * (j % PER + 1))) & MASK);
+    const uint32_t p = T16<DT>::pack2(__builtin_fmaf(q0, s, b), __builtin_fmaf(q1, s, b));
+    v[j] = T16<DT>::to_f32((uint16_t)p);
+    v[j + 1] = T16<DT>::to_f32((uint16_t)(p >> 16));
+  }
+}
+
 // The `BITS` bytes of octet o (bitstream of 8 codes, lowest code lowest).
 template <int BITS>
 __device__ __forceinline__ void store_octet(uint8_t* wq, int64_t o, uint64_t bitsv) {
@@ -162,8 +189,15 @@ __device__ __forceinline__ void codes16(const float v[16], float scale, float bi
 // scales are of ordinary size takes plain minima (v_med3 with an infinity)
 // and divides by a reciprocal; two octets per thread share the four divisions
 // of a group's scale.  Any other wave runs every operation as written above.
-template <int DT, int BITS, int GS>
+//
+// SB 4 or 8 (16-bit DT): w holds SB-bit codes in groups of 8 << sshift codes with
+// scales ss and biases sb, and the values are T(float(s) * q + float(b)), as
+// dequantizing first gives them: one pass over the codes instead of two
+// kernels with the dequantized weights in memory between them.
+template <int DT, int BITS, int GS, int SB = 0>
 __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ w,
+                                                       const uint16_t* __restrict__ ss,
+                                                       const uint16_t* __restrict__ sb, int sshift,
                                                        uint8_t* __restrict__ wq,
                                                        void* __restrict__ scales,
                                                        void* __restrict__ biases, int64_t octets) {
@@ -177,8 +211,13 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
     const bool live = o < octets;
     float v[16];
     if (live) {
-      load_octet<DT>(w, o, v);
-      load_octet<DT>(w, o + 1, v + 8);
+      if constexpr (SB == 0) {
+        load_octet<DT>(w, o, v);
+        load_octet<DT>(w, o + 1, v + 8);
+      } else {
+        load_codes16<DT, SB>(w, T16<DT>::to_f32(ss[o >> sshift]),
+                             T16<DT>::to_f32(sb[o >> sshift]), o, v);
+      }
     } else {
 #pragma unroll
       for (int j = 0; j < 16; ++j) v[j] = 0.f;
@@ -306,8 +345,31 @@ template <int DT, int BITS, int GS>
 struct QuantizeRun {
   static int run(const void* w, uint32_t* wq, void* s, void* b, int64_t octets, hipStream_t st) {
     hipLaunchKernelGGL((quantize_kernel<DT, BITS, GS>), dim3(octet_grid(octets / 2)), dim3(256), 0,
-                       st, w, reinterpret_cast<uint8_t*>(wq), s, b, octets);
+                       st, w, (const uint16_t*)nullptr, (const uint16_t*)nullptr, 0,
+                       reinterpret_cast<uint8_t*>(wq), s, b, octets);
     return 0;
+  }
+};
+
+template <int DT, int BITS, int GS>
+struct RequantizeRun {
+  static int run(const uint32_t* w, const void* ss, const void* sb, int sgs, int sbits,
+                 uint32_t* wq, void* s, void* b, int64_t octets, hipStream_t st) {
+    if constexpr (DT == kF32) {
+      return kStatusUnsupported;
+    } else {
+      const int shift = sgs == 32 ? 2 : sgs == 64 ? 3 : 4;   // octets per source group
+      auto go = [&](auto c) {
+        hipLaunchKernelGGL((quantize_kernel<DT, BITS, GS, decltype(c)::value>),
+                           dim3(octet_grid(octets / 2)), dim3(256), 0, st, w,
+                           (const uint16_t*)ss, (const uint16_t*)sb, shift,
+                           reinterpret_cast<uint8_t*>(wq), s, b, octets);
+      };
+      if (sbits == 4) go(std::integral_constant<int, 4>{});
+      else if (sbits == 8) go(std::integral_constant<int, 8>{});
+      else return kStatusUnsupported;
+      return 0;
+    }
   }
 };
 
@@ -326,6 +388,13 @@ struct DequantBitsRun {
 int launch_quantize(const void* w, uint32_t* wq, void* scales, void* biases, int64_t N,
                     int64_t K, int group_size, int bits, int dtype, hipStream_t st) {
   return by_format<QuantizeRun>(dtype, bits, group_size, w, wq, scales, biases, N * K / 8, st);
+}
+
+int launch_requantize(const uint32_t* w, const void* src_scales, const void* src_biases,
+                      int src_group_size, int src_bits, uint32_t* wq, void* scales, void* biases,
+                      int64_t N, int64_t K, int group_size, int bits, int dtype, hipStream_t st) {
+  return by_format<RequantizeRun>(dtype, bits, group_size, w, src_scales, src_biases,
+                                  src_group_size, src_bits, wq, scales, biases, N * K / 8, st);
 }
 
 int launch_dequantize_bits(const uint32_t* wq, const void* scales, const void* biases, void* out,

@@ -180,6 +180,11 @@ int launch_swiglu(const void* g, const void* u, void* out, int64_t n, int dtype,
 // outside bits {2,3,4,5,6,8} x group {32,64,128} x dtype {bf16,f16,f32}.
 int launch_quantize(const void* w, uint32_t* wq, void* scales, void* biases, int64_t N,
                     int64_t K, int group_size, int bits, int dtype, hipStream_t st);
+
+// The same from 4- or 8-bit codes of 16-bit dtype DT, dequantized to DT first.
+int launch_requantize(const uint32_t* w, const void* src_scales, const void* src_biases,
+                      int src_group_size, int src_bits, uint32_t* wq, void* scales, void* biases,
+                      int64_t N, int64_t K, int group_size, int bits, int dtype, hipStream_t st);
 int launch_dequantize_bits(const uint32_t* wq, const void* scales, const void* biases, void* out,
                            int64_t N, int64_t K, int group_size, int bits, int dtype,
                            hipStream_t st);

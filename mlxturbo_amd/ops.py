@@ -160,6 +160,31 @@ def quantize(w: torch.Tensor, group_size: int = 64, bits: int = 4, mode: str = "
     return wq, scales, biases
 
 
+def _requantize(w, scales, biases, from_group_size: int, from_bits: int, group_size: int,
+                bits: int):
+    """``quantize(dequantize(w, scales, biases))`` in one kernel, bit for bit
+    (mq_requantize), or None where that kernel does not apply: codes of other
+    widths than 4 and 8 bits, float32, or arguments the two operators refuse."""
+    if (from_bits not in (4, 8) or bits not in _BITS or group_size not in _GROUP_SIZES
+            or biases is None or scales.dtype not in (torch.bfloat16, torch.float16)):
+        return None
+    dev = _require_gpu(w, scales, biases)
+    K = _check_quant(w, scales, biases, from_group_size, from_bits)
+    N = math.prod(w.shape[:-1])
+    if not N or not K or K % group_size:
+        return None
+    lead = tuple(w.shape[:-1])
+    wq = torch.empty((*lead, K * bits // 32), dtype=torch.uint32, device=dev)
+    s = torch.empty((*lead, K // group_size), dtype=scales.dtype, device=dev)
+    b = torch.empty_like(s)
+    w_, s_, b_ = _aligned(w), _aligned(scales), _aligned(biases)
+    rc = _lib.lib().mq_requantize(w_.data_ptr(), s_.data_ptr(), b_.data_ptr(), from_group_size,
+                                  from_bits, wq.data_ptr(), s.data_ptr(), b.data_ptr(), N, K,
+                                  group_size, bits, _DTYPE_CODE[s.dtype], _stream_ptr(wq))
+    _lib.check(rc, "requantize")
+    return wq, s, b
+
+
 def dequantize(w: torch.Tensor, scales: torch.Tensor, biases: Optional[torch.Tensor] = None,
                group_size: int = 64, bits: int = 4, mode: str = "affine") -> torch.Tensor:
     """``mx.dequantize``: ``T(float(s)*q + float(b))`` bit-exact, dtype of

@@ -21,6 +21,7 @@ from typing import Dict, Iterable, Optional, Tuple
 
 import torch
 
+from . import ops
 from .nn import QuantizedLinear
 
 CLASSES = ("gdn", "hc", "attn", "head", "router", "shared")
@@ -45,6 +46,16 @@ def requantize(layer, bits: int, group_size: int = 64) -> QuantizedLinear:
     quantization, as rebit.py:96-120 does); a ``torch.nn.Linear`` or any
     module with a float ``weight`` is quantized directly.  ``bias`` is kept."""
     if isinstance(layer, QuantizedLinear):
+        # both steps in one pass over the codes where the kernel takes them
+        # (5120 x 17408, 8 to 4 bits: 47.6 us against 96.0 for the two)
+        if (layer.mode == "affine" and layer.weight.is_cuda
+                and type(layer).dequantized_weight is QuantizedLinear.dequantized_weight):
+            q = ops._requantize(layer.weight, layer.scales, layer.biases, layer.group_size,
+                                layer.bits, group_size, bits)
+            if q is not None:
+                bias = layer.bias
+                return QuantizedLinear(*q, bias=None if bias is None else bias.detach(),
+                                       group_size=group_size, bits=bits)
         w = layer.dequantized_weight()
     else:
         w = layer.weight.detach()

@@ -61,3 +61,34 @@ def test_quantize_routes(bits, gs, rows, dtype):
     for g, e in zip(got[1:], want[1:]):
         e = O.to_f32(e, dtype)
         np.testing.assert_array_equal(g.float().cpu().numpy(), e)   # NaN equals NaN
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("from_bits, from_gs, bits, gs, N, K", [
+    (8, 64, 4, 64, 130, 640), (8, 128, 4, 32, 33, 384), (8, 32, 2, 128, 7, 1152),
+    (4, 32, 8, 64, 65, 192), (4, 64, 3, 32, 40, 320), (4, 128, 6, 64, 1, 128),
+    (8, 64, 5, 128, 63, 256), (4, 64, 4, 64, 257, 64),
+])
+def test_requantize_is_dequantize_then_quantize(from_bits, from_gs, bits, gs, N, K, dtype):
+    """One pass over the codes: the bytes of the two operators, with scales of
+    either sign, out of the reciprocal's range, infinite and NaN."""
+    g = torch.Generator(device="cuda").manual_seed(N + K + bits)
+    w = torch.randint(-2**31, 2**31, (N, K * from_bits // 32), generator=g, device="cuda",
+                      dtype=torch.int64).to(torch.int32).view(torch.uint32)
+    s = torch.randn((N, K // from_gs), generator=g, device="cuda")
+    b = torch.randn((N, K // from_gs), generator=g, device="cuda") * 8
+    if N > 1:
+        s[0] = 1e-30
+        s[N // 2, 0] = float("inf")
+        b[N // 3, 0] = float("nan")
+        s[N - 1] *= 1e4 if dtype == "float16" else 1e34
+    s, b = s.to(TORCH_DTYPE[dtype]), b.to(TORCH_DTYPE[dtype])
+    kw = dict(group_size=gs, bits=bits)
+    got = mq.ops._requantize(w, s, b, from_gs, from_bits, gs, bits)
+    want = mq.quantize(mq.dequantize(w, s, b, group_size=from_gs, bits=from_bits), **kw)
+    for x, y in zip(got, want):
+        assert x.shape == y.shape and x.dtype == y.dtype
+        assert torch.equal(x.view(torch.int32) if x.dtype == torch.uint32 else x.view(torch.int16),
+                           y.view(torch.int32) if y.dtype == torch.uint32 else y.view(torch.int16))
+    assert mq.ops._requantize(w, s, b, from_gs, from_bits, gs, 7) is None
+    assert mq.ops._requantize(w, s.float(), b.float(), from_gs, from_bits, gs, bits) is None
