@@ -56,15 +56,18 @@ uint64_t mq_launch_count(void);
 /*
  * Row identity across call widths (process-wide, default 0).  One-row
  * calls (M = 1) normally run their own kernel, whose sums are rounded in a
- * different order from the 2..32-row kernels': each row is within the
- * output tolerance of both, not bit-identical to the same row computed in
- * a wider call.  With on != 0, one-row calls run the 2..32-row kernel
- * family, so a row's result does not depend on how many rows the call has
+ * different order from the 2..32-row kernels', and calls of 17..32 rows the
+ * wide tile where that is the cheaper: each row is within the output
+ * tolerance of all of them, not bit-identical to the same row computed in
+ * a call of another width.  With on != 0, calls of 1 to 32 rows all run the
+ * 2..32-row kernel family, so a row's result does not depend on how many of
+ * these rows the call has
  * (decode vs. speculative verify).  The reference keeps this property with
  * its opt-in small-M route: rows of an M = 2..8 call bit-identical to the
  * M = 1 call (kernels/qmv_small_m.py:289-307, dispatch.py:337-347).
  * Returns the previous setting.  Not for calls running concurrently with a
- * change of the setting.
+ * change of the setting; workspaces are to be sized under the setting that
+ * the call runs under.
  */
 int mq_set_row_identity(int on);
 

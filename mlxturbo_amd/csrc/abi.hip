@@ -16,7 +16,7 @@ namespace {
 
 thread_local std::string g_last_error;
 std::atomic<uint64_t> g_launches{0};
-// one-row calls on the 2..32-row kernel family (mq_set_row_identity)
+// calls of 1..32 rows all on the 2..32-row kernel family (mq_set_row_identity)
 std::atomic<int> g_row_identity{0};
 
 int fail(int code, const char* fmt, ...) {
@@ -222,7 +222,8 @@ int mq_requantize(const uint32_t* w, const void* scales, const void* biases, int
 size_t mq_quantized_matmul_workspace_size(int64_t M, int64_t N, int64_t K, int group_size,
                                           int bits) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size) return 0;
-  return mq::qmm_workspace_bytes(M, N, K, bits, group_size, mq::device_cu_count());
+  return mq::qmm_workspace_bytes(M, N, K, bits, group_size, mq::device_cu_count(),
+                                 g_row_identity.load(std::memory_order_relaxed) != 0);
 }
 
 int mq_quantized_matmul_ws(const void* x, const uint32_t* w, const void* scales,
@@ -244,10 +245,11 @@ int mq_quantized_matmul_ws(const void* x, const uint32_t* w, const void* scales,
   if (M == 0 || N == 0) return MQ_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(hip_stream);
   const int cus = mq::device_cu_count();
+  const bool row_identity = g_row_identity.load(std::memory_order_relaxed) != 0;
   // K splits only when the caller's workspace holds the planned partials
-  const size_t need = mq::qmm_workspace_bytes(M, N, K, bits, group_size, cus);
+  const size_t need = mq::qmm_workspace_bytes(M, N, K, bits, group_size, cus, row_identity);
   const bool split_ok = workspace && need && workspace_bytes >= need;
-  if (mq::wide_route(M, N, K, bits, group_size, cus, split_ok)) {
+  if (mq::wide_route(M, N, K, bits, group_size, cus, split_ok, row_identity)) {
     int nl = 0;
     rc = dispatch_16<mq::WideLaunch>(dtype, bits, group_size, x, w, scales, biases, out, M, N, K,
                                      split_ok ? workspace : nullptr,
@@ -260,7 +262,7 @@ int mq_quantized_matmul_ws(const void* x, const uint32_t* w, const void* scales,
     return MQ_OK;
   }
   int nl = 0;
-  if (M == 1 && !g_row_identity.load(std::memory_order_relaxed)) {
+  if (M == 1 && !row_identity) {
     rc = dispatch_16<mq::QuadLaunch>(dtype, bits, group_size, x, w, scales, biases, out, M, N, K,
                                      st, &nl);
     if (rc == 0) {

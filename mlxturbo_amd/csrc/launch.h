@@ -384,10 +384,12 @@ inline size_t skinny_split_bytes(int64_t M, int64_t N, int64_t K, int bits, int 
 // in one launch at x1.5 (two 16-row A tiles per weight fragment: M=17/24/32
 // 22.0/21.6/21.1 us, one process); the wide tile by wide_plan (K=5120 N=17408:
 // M=96 from the third row of tiles on, 40 us at 128 rows against 66 in 32-row
-// launches).  split_ok: a workspace is available for K splits.
-inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus,
-                       bool split_ok) {
-  if (!wide_eligible(M, N, K, bits, gs)) return false;
+// launches).  split_ok: a workspace is available for K splits.  row_identity
+// (mq_set_row_identity): up to 32 rows on the skinny family for every matrix,
+// whose rows then have the bits of a one-row call.
+inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus, bool split_ok,
+                       bool row_identity) {
+  if (!wide_eligible(M, N, K, bits, gs) || (row_identity && M <= 32)) return false;
   const int sx = skinny_shared_x_rows(N, K, bits, gs, cus);
   if (M <= 64 && (sx == 32 || (split_ok && skinny_split_slices(M, N, K, bits, gs)))) return false;
   const double wbytes = (double)N * (double)K * bits / 8.0;
@@ -419,8 +421,10 @@ inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cu
 
 // Workspace bytes of quantized_matmul (K splits of the wide kernel or of the
 // split skinny launches), 0 when the chosen plan needs none.
-inline size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus) {
-  if (!wide_route(M, N, K, bits, gs, cus, true)) return skinny_split_bytes(M, N, K, bits, gs);
+inline size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus,
+                                  bool row_identity) {
+  if (!wide_route(M, N, K, bits, gs, cus, true, row_identity))
+    return skinny_split_bytes(M, N, K, bits, gs);
   return wide_workspace_bytes(wide_plan(M, N, K, cus), M, N);
 }
 

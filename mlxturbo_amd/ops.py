@@ -1183,16 +1183,19 @@ def launch_count() -> int:
 
 
 def set_row_identity(on: bool) -> bool:
-    """Run one-row ``quantized_matmul`` calls on the 2..32-row kernel family,
-    so every output row is bit-identical whatever the number of rows in the
-    call (a decode step and a speculative verify of the same token agree bit
-    for bit).  Off by default: one-row calls then take their own faster
-    kernel, within the output tolerance of the wide rows but rounded in
-    another order.  The reference's counterpart is its opt-in small-M route,
+    """Run every ``quantized_matmul`` call of 1 to 32 rows on the 2..32-row
+    kernel family, so every output row is bit-identical whatever the number of
+    rows in the call (a decode step and a speculative verify of the same token
+    agree bit for bit).  Off by default: one-row calls then take their own
+    faster kernel, and calls of 17-32 rows the wide tile where that is the
+    cheaper, within the output tolerance of each other but rounded in another
+    order.  The reference's counterpart is its opt-in small-M route,
     whose rows of 2..8-row calls are bit-identical to the one-row call
     (kernels/qmv_small_m.py:289-307, dispatch.py:337-347).  Process-wide;
     returns the previous setting."""
-    return bool(_lib.lib().mq_set_row_identity(1 if on else 0))
+    prev = bool(_lib.lib().mq_set_row_identity(1 if on else 0))
+    _QMM_WS_BYTES.clear()                        # the sizes follow the route
+    return prev
 
 
 @contextlib.contextmanager

@@ -16,6 +16,7 @@ import torch
 
 import mlxturbo_amd as mq
 from mlxturbo_amd import _lib
+from mlxturbo_amd.nn import QuantizedLinear
 from oracle import oracle as O
 from qmm_helpers import (act, bits16, from_dev, quantized, random_packed, to_dev, uniform_routing,
                          zipf_routing)
@@ -197,6 +198,29 @@ def test_row_identity_switch(N, K, bits):
     one = mq.quantized_matmul(xd[3:4], *args, bits=bits)
     _check(one[:, torch.from_numpy(cols).cuda()],
            O.quantized_matmul_ref(x[3:4], w[cols], s[cols], b[cols], 64, bits))
+
+
+@pytest.mark.parametrize("N, K, bits, gs", [
+    (17408, 5120, 4, 32), (17408, 5120, 8, 128), (5120, 17408, 4, 128), (5120, 17408, 8, 128),
+    (12288, 4096, 4, 32), (10240, 5120, 4, 64), (300, 2048, 4, 128), (1000, 4160, 8, 32),
+])
+def test_row_identity_up_to_32_rows(N, K, bits, gs):
+    """The switch holds for every group size and matrix up to 32 rows, where the
+    wide tile would otherwise take some of the calls: every row has the bits of
+    its own one-row call."""
+    rng = np.random.default_rng(N + K + bits + gs)
+    w, s, b = random_packed(rng, N, K, gs, bits)
+    args = (to_dev(w), to_dev(s, "bfloat16"), to_dev(b, "bfloat16"))
+    xd = to_dev(act(rng, (32, K), scale=0.1), "bfloat16")
+    kw = dict(group_size=gs, bits=bits)
+    layer = QuantizedLinear(*args, **kw)
+    with mq.row_identity():
+        one = np.concatenate([bits16(mq.quantized_matmul(xd[m:m + 1], *args, **kw))
+                              for m in range(32)])
+        for M in (2, 16, 17, 20, 24, 32):
+            np.testing.assert_array_equal(bits16(mq.quantized_matmul(xd[:M], *args, **kw)),
+                                          one[:M])
+            np.testing.assert_array_equal(bits16(layer(xd[:M])), one[:M])
 
 
 def _qmm_abi(xd, wd, sd, bd, M, N, K, gs=64, bits=4):

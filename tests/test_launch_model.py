@@ -1,0 +1,29 @@
+"""Which kernel family a quantized_matmul call runs, from the library's own
+launch model (launch_model.cpp), without a GPU."""
+
+import itertools
+
+import pytest
+
+import host_program
+
+SHAPES = [(17408, 5120), (5120, 17408), (12288, 4096), (10240, 5120), (2048, 1024), (300, 2048),
+          (36000, 1024), (1000, 4160), (248320, 5120)]
+
+
+def routes(cases):
+    """(route, tile rows, splits, unit) of cases (M, N, K, bits, gs, ws, row identity)."""
+    out = host_program.run("launch_model.cpp", [" ".join(map(str, map(int, c))) for c in cases])
+    assert len(out) == len(cases)
+    return [tuple(map(int, line.split())) for line in out]
+
+
+@pytest.mark.parametrize("bits, gs", list(itertools.product([4, 8], [32, 64, 128])))
+def test_row_identity_keeps_one_family(bits, gs):
+    cases = [(M, N, K, bits, gs, ws, 1) for (N, K) in SHAPES if K % gs == 0
+             for M in (1, 2, 16, 17, 20, 24, 31, 32) for ws in (0, 1)]
+    assert {r[0] for r in routes(cases)} == {0}
+    # without the switch, and past 32 rows, the cheaper family
+    assert any(r[0] for r in routes([c[:6] + (0,) for c in cases]))
+    assert all(r[0] for r in routes([(512, N, K, bits, gs, 1, 1) for N, K in SHAPES
+                                     if K % gs == 0 and K % 64 == 0]))
