@@ -161,14 +161,10 @@ inline int wide_launch_bm(const void* x, const uint32_t* w, const void* s, const
                        st, (const uint16_t*)x, w, (const uint16_t*)s, (const uint16_t*)b,
                        (uint16_t*)out, part, (int)M, (int)N, (int)K, splits);
   };
-  if constexpr (BM == 256) {
-    go(std::integral_constant<int, 4>{});
-  } else {
-    const int u = wide_unit(K, s, b);
-    if (u == 4) go(std::integral_constant<int, 4>{});
-    else if (u == 2 || BM == 128) go(std::integral_constant<int, 2>{});
-    else if constexpr (BM != 128) go(std::integral_constant<int, 1>{});
-  }
+  const int u = wide_unit(K, s, b);
+  if (u == 4) go(std::integral_constant<int, 4>{});
+  else if (u == 2) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 1>{});
   if (splits > 1) {
     const int64_t MN = M * N;
     const dim3 rg((unsigned)((MN + 1023) / 1024));
@@ -190,14 +186,9 @@ int WideLaunch<DT, BITS, GS>::run(const void* x, const uint32_t* w, const void* 
   if (K * 2 * 256 >= ((int64_t)1 << 31) || M > ((int64_t)1 << 31) / 256 * 256)
     return kStatusUnsupported;
   const int cus = device_cu_count();
-  // the scales' address may allow fewer steps per load than the plan takes (K
-  // and the matrix say the rest): a tile height that has such a kernel
-  const int u = wide_unit(K, s, b);
-  WidePlan plan = wide_plan(M, N, K, cus, 16);
+  WidePlan plan = wide_plan(M, N, K, BITS, cus);
   if (plan.splits > 1 && (!ws || ws_bytes < wide_workspace_bytes(plan, M, N)))
-    plan = wide_plan(M, N, K, cus, 1);
-  if (u < 4 && plan.bm == 256) plan.bm = 192;
-  if (u < 2 && plan.bm == 128) plan.bm = 192;
+    plan = wide_plan(M, N, K, BITS, cus, 1);
   const int splits = plan.splits;
   *nlaunch += splits > 1 ? 2 : 1;
   switch (plan.bm) {

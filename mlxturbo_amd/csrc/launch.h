@@ -241,56 +241,70 @@ inline int device_cu_count() {
 }
 
 // Launch plan of the wide kernel (dense.cuh): row-tile height and K split, the
-// pair of least cost by a model fitted to measurements at K=5120 N=17408 and
-// K=17408 N=5120, M=64..8192:
-//  * a tile takes c0 (launch, first loads, stores) plus t per 64-code step;
-//    one alone 5.4 / 7.6 / 8.8 / 11.6 us plus 0.57 / 0.64 / 0.76 / 0.97 us
-//    (BM = 64 .. 256), with every CU busy the t below (M=1024, K=5120:
-//    192-row tiles 91 us a round, 256-row ones 106, 128-row ones 67);
+// pair of least cost by a model fitted to measurements:
+//  * a tile takes c0 (launch, first loads, stores) plus t per 64-code step
+//    with every CU busy;
 //  * a round of one tile per CU costs the same however few CUs it fills, but
 //    over many rounds power holds the clock, and idle CUs leave it to the
-//    others: then tiles / CUs rounds at tp per step count (K=5120: M=8192
-//    1128 us in 8.5 rounds of 256-row tiles, 1187 in 11.4 of 192-row ones;
-//    M=2048 347 in 2.1 and 302 in 2.9);
-//  * K splits sum into float [M, N] planes that a second kernel adds, 3 us
-//    plus (8 S + 2) M N bytes written and read at ~7 TB/s (they stay in the
-//    last-level cache): M=128 K=5120 39.9 us with 3 splits of 128-row tiles
-//    against 58.9 with one; M=256 K=17408 63.5 with 8 of 256-row tiles.
-// Scales are loaded for 4, 2 or 1 steps at a time (wide_unit), which K and
-// their address must allow; 256-row tiles exist for 4 and 128-row ones for 4
-// and 2 (the shorter loads' kernels of these heights do not fit the registers
-// or gain nothing).
+//    others: then tiles / CUs rounds at tp per step count (K=5120 N=17408, 4
+//    bits: M=8192 1128 us in 8.5 rounds of 256-row tiles, 1187 in 11.4 of
+//    192-row ones; M=2048 347 in 2.1 and 302 in 2.9);
+//  * K splits sum into float [M, N] planes that a second kernel adds, in 3 us
+//    (whole 256s of K) or 6 (otherwise) plus (8 S + 2) M N bytes written and read at ~7 TB/s
+//    (they stay in the last-level cache): M=128 K=5120 39.9 us with 3 splits of
+//    128-row tiles against 58.9 with one; M=256 K=17408 63.5 with 8 of 256-row
+//    tiles.
+// A step costs more where scales are loaded for 2 steps or 1 at a time
+// (wide_unit), and with 8-bit codes there, so each has constants of its own,
+// fitted to every height and split of 14 row counts (17 .. 2048) on six
+// matrices each.
 struct WidePlan {
   int bm = 256, splits = 1;
   double cost_us = 0.0;
 };
 
+// Steps per load of scales: what K, and the address where it is given, allow.
 inline int wide_unit(int64_t K, const void* s = nullptr, const void* b = nullptr) {
   if (((uintptr_t)s | (uintptr_t)b) % 4) return 1;
   return K % 256 == 0 ? 4 : K % 128 == 0 ? 2 : 1;
 }
 
-inline WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int cus, int max_splits = 16) {
+struct WideTileUs {
+  double c0, t, tp;
+};
+
+// tile heights 64, 128, 192, 256
+inline const WideTileUs* wide_tile_us(int bits, int unit) {
+  static const WideTileUs us[2][3][4] = {
+      {{{1.50, 0.82, 1.24}, {3.69, 1.02, 1.13}, {4.15, 1.21, 1.47}, {9.89, 1.36, 1.61}},
+       {{2.09, 0.71, 0.85}, {4.96, 0.83, 0.96}, {4.92, 1.12, 1.25}, {8.84, 1.34, 1.56}},
+       {{5.4, 0.59, 0.62}, {7.6, 0.72, 0.83}, {8.8, 1.06, 1.18}, {11.6, 1.24, 1.48}}},
+      {{{1.30, 0.96, 1.12}, {5.18, 1.16, 1.16}, {5.80, 1.35, 1.52}, {8.45, 1.51, 1.68}},
+       {{1.44, 0.98, 0.98}, {3.73, 1.11, 1.31}, {6.22, 1.23, 1.43}, {10.58, 1.38, 1.67}},
+       {{5.4, 0.59, 0.62}, {7.6, 0.72, 0.83}, {8.8, 1.06, 1.18}, {11.6, 1.24, 1.48}}}};
+  return us[bits == 8][unit >> 1];
+}
+
+inline WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int bits, int cus,
+                          int max_splits = 16) {
   const int64_t cols = (N + 255) / 256;
   const int unit = wide_unit(K);
   const int64_t nu = K / (64 * unit);
   const int bms[4] = {64, 128, 192, 256};
-  const double c0[4] = {5.4, 7.6, 8.8, 11.6};
-  const double t[4] = {0.59, 0.72, 1.06, 1.24};
-  const double tp[4] = {0.62, 0.83, 1.18, 1.48};
+  const WideTileUs* us = wide_tile_us(bits, unit);
+  const double sum_us = unit == 4 ? 3.0 : 6.0;
   WidePlan best;
   bool first = true;
   for (int sp = 1; sp <= max_splits; ++sp) {
     const double steps = (double)(unit * ((nu + sp - 1) / sp));
     if (sp > 1 && steps < 8) break;             // at least 8 k-steps per split
     for (int i = 3; i >= 0; --i) {
-      if ((bms[i] == 256 && unit < 4) || (bms[i] == 128 && unit < 2)) continue;
       const int64_t tiles = cols * ((M + bms[i] - 1) / bms[i]) * sp;
       const double rounds = (double)((tiles + cus - 1) / cus);
-      double cost = rounds * (c0[i] + t[i] * steps);
-      const double held = (double)tiles / cus * (tp[i] * steps) + c0[i];
+      double cost = rounds * (us[i].c0 + us[i].t * steps);
+      const double held = (double)tiles / cus * (us[i].tp * steps) + us[i].c0;
       if (held > cost) cost = held;
-      if (sp > 1) cost += 3.0 + (8.0 * sp + 2.0) * (double)M * (double)N / 7.0e6;
+      if (sp > 1) cost += sum_us + (8.0 * sp + 2.0) * (double)M * (double)N / 7.0e6;
       if (first || cost < best.cost_us) {
         best.bm = bms[i];
         best.splits = sp;
@@ -393,7 +407,7 @@ inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cu
   const int sx = skinny_shared_x_rows(N, K, bits, gs, cus);
   if (M <= 64 && (sx == 32 || (split_ok && skinny_split_slices(M, N, K, bits, gs)))) return false;
   const double wbytes = (double)N * (double)K * bits / 8.0;
-  const double wide_us = wide_plan(M, N, K, cus, split_ok ? 16 : 1).cost_us;
+  const double wide_us = wide_plan(M, N, K, bits, cus, split_ok ? 16 : 1).cost_us;
   const double one = 3.0 + wbytes / 3.6e6;
   const bool shared_x = sx > 0;
   double skinny_us = 0.0;
@@ -425,7 +439,7 @@ inline size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int
                                   bool row_identity) {
   if (!wide_route(M, N, K, bits, gs, cus, true, row_identity))
     return skinny_split_bytes(M, N, K, bits, gs);
-  return wide_workspace_bytes(wide_plan(M, N, K, cus), M, N);
+  return wide_workspace_bytes(wide_plan(M, N, K, bits, cus), M, N);
 }
 
 // gather_qmm: up to kGatherFusedMaxP pairs are grouped by expert inside the

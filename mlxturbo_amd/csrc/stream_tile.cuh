@@ -138,8 +138,8 @@ struct StreamLds {
 // GLU: the wave's blocks are rows 32 w .. 32 w + 31 of two matrices (w and
 // w2) instead.  U: steps per load of scales, 4, 2 or 1: K in whole 64 U codes,
 // kt0 and nk in whole U steps, scales and biases 4-byte aligned where U > 1.
-// One 2-byte load per step and block cost 1.3-1.6x (M=512 K=5120 N=17408, 192
-// rows: 122 us against 92 with U = 4).
+// A step of a 192-row tile takes 1.1 us at U = 1 and 0.96 at 2 against 0.86 at
+// 4 (4 bits; launch.h wide_tile_us).
 // put(acc): the sums, acc[i][j][e] of tile row 32 i + (lane & 31) and weight
 // row 8 (e / 4) + 4 (lane >> 5) + e % 4 of block j; put_block(i, j, acc) the
 // same of one block (plain route).  Both are called by every wave after the
@@ -302,10 +302,6 @@ __device__ __forceinline__ void stream_tile(
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-  // Loads per step that the waits before the barriers may count on.  The loop
-  // leaves in its middle where U < 4, and the compiler then moves loads into
-  // registers past the exits (never those into LDS): only the latter count.
-  constexpr int NVM = U == 4 ? DM + 2 * WB : DM;
   // load v of step kn into stage S
   auto load = [&](int kn, auto sc, auto vc) {
     constexpr int v = decltype(vc)::value;
@@ -349,7 +345,8 @@ __device__ __forceinline__ void stream_tile(
   });
   static_for<0, 16>([&](auto xc) { bpiece(I0{}, I0{}, I0{}, xc); });
 
-  auto step = [&](int kt, auto uc) {
+  // nvm: the loads of one step that the wait before the barrier may count on
+  auto step = [&](int kt, auto uc, auto nvm) {
     constexpr int u = decltype(uc)::value;
     using S = std::integral_constant<int, u>;
     using N1 = std::integral_constant<int, (u + 1) & 3>;
@@ -370,29 +367,41 @@ __device__ __forceinline__ void stream_tile(
       if constexpr (decltype(tc)::value == 0) group(N1{}, I0{});
       if constexpr (decltype(tc)::value == NS / 2) group(N1{}, I1{});
     });
-    barrier(std::integral_constant<int, 2 * NVM>{});
+    barrier(std::integral_constant<int, 2 * decltype(nvm)::value>{});
     g[0] = gn[0];
     g[1] = gn[1];
     if constexpr ((u + 1) % U == 0) take(std::integral_constant<int, (u + 1) / U % RU>{});
     substep(I1{}, N1{}, I0{}, [&](auto) {});
   };
+  // Whole fours of steps in a loop that is left at its end alone: left in its
+  // middle, the compiler moves loads into registers (not those into LDS) past
+  // the exits, to the end of the body, and the weights no longer run ahead.
+  // The up to three steps of a K that is not whole fours come after it, where
+  // the waits count the loads into LDS alone for the same reason.
+  using Counted = std::integral_constant<int, NL>;
+  using Sure = std::integral_constant<int, DM>;
+  const int n4 = U == 4 ? nk : nk & ~3;
   int kt = 0;
-  do {                                          // no branch that loads could sink past
-    step(kt, I0{});
-    if constexpr (U == 1) {
-      if (kt + 1 >= nk) break;
+  if (U == 4 || n4 > 0) {
+    do {
+      step(kt, I0{}, Counted{});
+      step(kt + 1, I1{}, Counted{});
+      step(kt + 2, I2{}, Counted{});
+      step(kt + 3, I3{}, Counted{});
+      kt += 4;
+    } while (kt < n4);
+  }
+  if constexpr (U < 4) {
+    if (kt < nk) {
+      step(kt, I0{}, Sure{});
+      if (U == 2 || kt + 1 < nk) {
+        step(kt + 1, I1{}, Sure{});
+        if constexpr (U == 1) {
+          if (kt + 2 < nk) step(kt + 2, I2{}, Sure{});
+        }
+      }
     }
-    step(kt + 1, I1{});
-    if constexpr (U < 4) {
-      if (kt + 2 >= nk) break;
-    }
-    step(kt + 2, I2{});
-    if constexpr (U == 1) {
-      if (kt + 3 >= nk) break;
-    }
-    step(kt + 3, I3{});
-    kt += 4;
-  } while (kt < nk);
+  }
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
   asm volatile("" ::: "memory");

@@ -1,6 +1,8 @@
 """The 256-column MFMA tile whose weights go from memory through registers into
 MFMA operands: the wide kernel of quantized_matmul and the thin grouped kernel
-of 8-bit banks, at the edges of its rows, columns, k-steps and scale loads.
+of 8-bit banks, at the edges of its rows, columns, k-steps and scale loads, and
+at every tile height (test_launch_model.py checks on the CPU that TALL's shapes
+are planned as written).
 
 References are float64 products of the dequantized weights, rounded to the
 output type.  Tolerance: a float32 sum of K terms is off by about sqrt(K) 2^-24
@@ -41,13 +43,53 @@ def _shifted(t):
     (127, 255, 320, 4, 64, BF16),      # steps of scales one by one (K = 64 odd)
     (129, 1000, 640, 8, 128, F16),     # two by two
     (193, 264, 1152, 4, 32, BF16),     # two groups per step, two by two
-    (257, 250, 512, 8, 32, F16),       # rows past a 256-row tile, four by four
+    (257, 250, 512, 8, 32, F16),       # one row past four tiles, four by four
     (300, 5121, 2048, 4, 128, BF16),   # N odd: stores of single values
     (96, 512, 4096, 8, 64, BF16),      # K split over workgroups
     (385, 768, 8192, 4, 64, F16),
     (1030, 513, 256, 4, 64, BF16),     # one round of four steps
 ])
 def test_wide_edges(M, N, K, bits, gs, dtype):
+    """Small matrices, all planned as 64-row tiles."""
+    _wide(M, N, K, bits, gs, dtype)
+
+
+# M, N, K, bits, group size, dtype; then the plan: rows of a tile, steps per load
+# of scales, whether K is split.  Odd N stores values one by one.
+TALL = [
+    (70, 40007, 192, 4, 64, BF16, 128, 1, False),     # three steps: no whole four
+    (200, 17408, 448, 8, 32, F16, 128, 1, False),     # one whole four and three
+    (70, 8200, 2880, 4, 32, BF16, 128, 1, True),      # eleven fours and one, split
+    (70, 40007, 384, 4, 64, BF16, 128, 2, False),
+    (70, 8200, 2944, 8, 128, BF16, 128, 2, True),
+    (200, 17408, 512, 4, 64, F16, 128, 4, False),
+    (70, 8200, 4096, 4, 32, BF16, 128, 4, True),
+    (450, 17413, 64, 4, 64, BF16, 192, 1, False),     # one step
+    (450, 17408, 320, 8, 32, F16, 192, 1, False),
+    (129, 8200, 2880, 4, 64, BF16, 192, 1, True),
+    (450, 17413, 128, 8, 64, BF16, 192, 2, False),
+    (450, 17408, 384, 4, 32, BF16, 192, 2, False),
+    (129, 8200, 2944, 8, 128, F16, 192, 2, True),
+    (385, 17408, 512, 4, 128, F16, 192, 4, False),
+    (129, 8200, 5120, 4, 64, BF16, 192, 4, True),
+    (600, 17413, 320, 4, 64, BF16, 256, 1, False),
+    (200, 17408, 2880, 8, 32, BF16, 256, 1, True),
+    (600, 17408, 384, 4, 128, F16, 256, 2, False),
+    (200, 17413, 4224, 8, 64, BF16, 256, 2, True),
+    (600, 17413, 512, 4, 64, BF16, 256, 4, False),
+    (200, 17408, 5120, 4, 128, BF16, 256, 4, True),
+]
+
+
+@pytest.mark.parametrize("M, N, K, bits, gs, dtype, bm, unit, split", TALL)
+def test_wide_heights(M, N, K, bits, gs, dtype, bm, unit, split):
+    """Tiles of 128, 192 and 256 rows, with scales loaded for four, two and one
+    steps, fours of steps with and without a rest; with the scales at an odd
+    address every height runs its one-step loads."""
+    _wide(M, N, K, bits, gs, dtype)
+
+
+def _wide(M, N, K, bits, gs, dtype):
     g, (w, s, b) = _quantized(N, K, bits, gs, dtype, M + N + K)
     x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
     ref = x.double() @ mq.dequantize(w, s, b, group_size=gs, bits=bits).double().T
@@ -55,6 +97,8 @@ def test_wide_edges(M, N, K, bits, gs, dtype):
     _check(out, ref)
     _check(out[-1:], ref[-1:])
     _check(out[:, -1:], ref[:, -1:])
+    for r in range(0, M, 64):                  # a wrong tile shows in its own rows
+        _check(out[r:r + 64], ref[r:r + 64])
     # scales at an odd address; the C entry has no workspace, so no K split
     ss, sb = _shifted(s), _shifted(b)
     got = torch.full_like(out, float("nan"))
@@ -62,7 +106,8 @@ def test_wide_edges(M, N, K, bits, gs, dtype):
         x.data_ptr(), w.data_ptr(), ss.data_ptr(), sb.data_ptr(), got.data_ptr(), M, N, K, gs,
         bits, 0 if dtype == BF16 else 1, 1, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
-    _check(got, ref)
+    for r in range(0, M, 64):
+        _check(got[r:r + 64], ref[r:r + 64])
 
 
 @pytest.mark.parametrize("bits", [8, 4])

@@ -6,6 +6,7 @@ import itertools
 import pytest
 
 import host_program
+from test_gpu_stream_tile import TALL
 
 SHAPES = [(17408, 5120), (5120, 17408), (12288, 4096), (10240, 5120), (2048, 1024), (300, 2048),
           (36000, 1024), (1000, 4160), (248320, 5120)]
@@ -27,3 +28,14 @@ def test_row_identity_keeps_one_family(bits, gs):
     assert any(r[0] for r in routes([c[:6] + (0,) for c in cases]))
     assert all(r[0] for r in routes([(512, N, K, bits, gs, 1, 1) for N, K in SHAPES
                                      if K % gs == 0 and K % 64 == 0]))
+
+
+def test_wide_heights_are_planned():
+    """The shapes of test_gpu_stream_tile.TALL run the tiles they are there for,
+    with the workspace; without it (and the scales at an odd address) every one
+    still runs the wide kernel."""
+    cases = [c[:5] for c in TALL]
+    for c, r in zip(TALL, routes([(*c, 1, 0) for c in cases])):
+        assert r == (1, c[6], r[2], c[7]) and (r[2] > 1) == c[8], (c, r)
+    assert {(r[0]) for r in routes([(*c, 0, 0) for c in cases])} == {1}
+    assert {c[6:8] for c in TALL} == set(itertools.product([128, 192, 256], [1, 2, 4]))
