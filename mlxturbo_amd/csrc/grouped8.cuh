@@ -10,10 +10,13 @@
 // tables, looked up after the first weights are issued), output rows scattered
 // back to pair order.  Bound by the weight stream: a lane's two 16-byte loads
 // per step and block make whole 64-byte pieces of 8-bit rows, three steps
-// ahead.  512 experts of H=2048, I=512, 301 tokens x top-8: gate/up 118 us,
-// down 65, against 127 and 75 of 8- and 4-wave workgroups that loaded two
-// steps ahead and staged x through registers (the same loads of 4-bit rows
-// are half as long and lost to them).
+// ahead.  Against 8- and 4-wave workgroups that loaded two steps ahead and
+// staged x through registers (top-8, even routing; the same loads of 4-bit rows
+// are half as long and lost to them): 128 experts of H=2048, I=768, 301 tokens
+// gate/up 125 -> 109 us, down 74 -> 60; 512 experts of H=2048, I=512, 301
+// tokens 260 -> 281 and 162 -> 162, 2048 tokens 293 -> 304 and 173 -> 178; 128
+// experts of H=1536, I=512, 1500 tokens 83 -> 101 (94 rows per expert, one
+// 128-row tile before) and 70 -> 59; over 26 layers 12% less time in the mean.
 #pragma once
 #include "stream_tile.cuh"
 
@@ -68,17 +71,10 @@ __global__ __launch_bounds__(256, 2) void qmm_grouped_thin8_kernel(
   const int t = threadIdx.x, lane = t & 63, lr = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int n0 = col * BN, ncols = min(BN, N - n0);
-  // tile row r (rows past the end: the last one) of pair perm[st0 + r / Mi]
-  auto pair_row = [&](int r, int& p, int& mi) {
-    r = min(r, rows - 1);
-    const int q = Mi == 1 ? r : r / Mi;
-    p = perm[st0 + q];
-    mi = r - q * Mi;
-  };
+  // tile row r: row r % Mi of pair perm[st0 + r / Mi]
   if (t < BM) {
-    int p, mi;
-    pair_row(t, p, mi);
-    s_orow[t] = t < rows ? p * Mi + mi : -1;
+    const int q = Mi == 1 ? t : t / Mi;
+    s_orow[t] = t < rows ? perm[st0 + q] * Mi + t - q * Mi : -1;
   }
   if (e >= E) {
     __syncthreads();
@@ -91,9 +87,9 @@ __global__ __launch_bounds__(256, 2) void qmm_grouped_thin8_kernel(
   const int64_t wrow = (int64_t)e * N + n0, G = K / GS, Kw = K / 4;
   const auto xr = wide_rsrc(x, (int64_t)B * Mi * K * 2);
   auto xrow_off = [&](int r) {
-    int p, mi;
-    pair_row(r, p, mi);
-    return (uint32_t)(((int64_t)x_batch(lhs, p, P, B) * Mi + mi) * K * 2);
+    if (r >= rows) return 0x80000000u;          // past the range: zeros, no memory access
+    const int q = Mi == 1 ? r : r / Mi, p = perm[st0 + q];
+    return (uint32_t)(((int64_t)x_batch(lhs, p, P, B) * Mi + r - q * Mi) * K * 2);
   };
   const bool vec = N % 8 == 0 && (uintptr_t)out % 16 == 0;
   auto glu = [&](float g, float u) {

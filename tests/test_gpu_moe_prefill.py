@@ -6,10 +6,10 @@ launch, one combine.
 Checked: the SwiGLU kernel against its torch composition bit for bit (bf16,
 fp16, ragged lengths, unaligned views); gathers over shared tables against
 the same gathers building their own, bit for bit, with hot experts (the
-two-row-class tables, whose 128-pair segments the down bank's 4-wave kernel
-runs as two 64-row tiles); the fused gate+up+SwiGLU launch against the two
-gathers and the SwiGLU pass, bit for bit (8- and 4-wave kernels, ragged
-column counts, fp16, 8-bit, out-of-range experts); the whole layer against
+two-class tables, whose 128-pair segments the thin kernels run as two 64-row
+tiles); the fused gate+up+SwiGLU launch against the two gathers and the SwiGLU
+pass, bit for bit (the thin kernels of 4- and 8-bit banks, ragged column
+counts, fp16, out-of-range experts); the whole layer against
 the sort path (sorted gathers, torch SwiGLU, unsort or combine) bit for bit,
 at config-4 size (2048 tokens x top-8 over 512 experts, hidden 2048,
 intermediate 512) and small banks, zipf and uniform routing; each gather of
@@ -77,9 +77,9 @@ def _bank(rng, E, N, K, mlx=False):
 
 @pytest.mark.parametrize("routing", ["zipf", "uniform"])
 def test_gathers_over_shared_tables(routing):
-    """gate (K=2048, 8-wave kernel, 128-row tiles for hot experts) and down
-    (K=512, 4-wave kernel, 128-pair segments as two 64-row tiles) over one
-    table build equal the gathers that build their own, bit for bit."""
+    """gate (K=2048) and down (K=512), the 128-pair segments of hot experts as
+    two 64-row tiles, over one table build equal the gathers that build their
+    own, bit for bit."""
     rng = np.random.default_rng(7 if routing == "zipf" else 8)
     E, T, top, H, I = 64, 512, 8, 2048, 512
     _, gate = _bank(rng, E, I, H)
@@ -104,8 +104,8 @@ def test_gathers_over_shared_tables(routing):
 
 
 @pytest.mark.parametrize("E, T, top, H, I, routing, dtype, bits", [
-    (64, 512, 8, 2048, 512, "zipf", "bfloat16", 4),     # 8 waves, 128-row tiles
-    (64, 512, 8, 1024, 256, "uniform", "bfloat16", 4),  # 4 waves, halves
+    (64, 512, 8, 2048, 512, "zipf", "bfloat16", 4),     # hot experts: pairs of tiles
+    (64, 512, 8, 1024, 256, "uniform", "bfloat16", 4),
     (48, 300, 4, 512, 200, "zipf", "bfloat16", 4),      # ragged column tile
     (64, 512, 8, 2048, 512, "zipf", "float16", 4),
     (64, 256, 8, 1024, 384, "uniform", "bfloat16", 8),
