@@ -250,14 +250,18 @@ inline int device_cu_count() {
 //    bits: M=8192 1128 us in 8.5 rounds of 256-row tiles, 1187 in 11.4 of
 //    192-row ones; M=2048 347 in 2.1 and 302 in 2.9);
 //  * K splits sum into float [M, N] planes that a second kernel adds, in 3 us
-//    (whole 256s of K) or 6 (otherwise) plus (8 S + 2) M N bytes written and read at ~7 TB/s
+//    (4 bits and whole 256s of K) or 6 (otherwise, where short calls of few
+//    tiles were measured too: K=1024 N=2048 M=512, 8 bits, 17.4 us split in
+//    two against 14.6) plus (8 S + 2) M N bytes written and read at ~7 TB/s
 //    (they stay in the last-level cache): M=128 K=5120 39.9 us with 3 splits of
 //    128-row tiles against 58.9 with one; M=256 K=17408 63.5 with 8 of 256-row
 //    tiles.
-// A step costs more where scales are loaded for 2 steps or 1 at a time
-// (wide_unit), and with 8-bit codes there, so each has constants of its own,
-// fitted to every height and split of 14 row counts (17 .. 2048) on six
-// matrices each.
+// A step costs more with 8-bit codes (twice the bytes) and where scales are
+// loaded for 2 steps or 1 at a time (wide_unit), so each has constants of its
+// own, fitted (all but the 4-bit, whole-256 ones) to every height and split of
+// 14 row counts (17 .. 2048) on six to eight matrices each; the plan so chosen
+// is 0.2% off the best one measured (geometric mean of 560 calls, 8% at most).  With the 4-bit, whole-256 constants for all, 8-bit
+// calls of 192 rows took 76 us where 65 is possible (K=5120 N=17408).
 struct WidePlan {
   int bm = 256, splits = 1;
   double cost_us = 0.0;
@@ -281,7 +285,7 @@ inline const WideTileUs* wide_tile_us(int bits, int unit) {
        {{5.4, 0.59, 0.62}, {7.6, 0.72, 0.83}, {8.8, 1.06, 1.18}, {11.6, 1.24, 1.48}}},
       {{{1.30, 0.96, 1.12}, {5.18, 1.16, 1.16}, {5.80, 1.35, 1.52}, {8.45, 1.51, 1.68}},
        {{1.44, 0.98, 0.98}, {3.73, 1.11, 1.31}, {6.22, 1.23, 1.43}, {10.58, 1.38, 1.67}},
-       {{5.4, 0.59, 0.62}, {7.6, 0.72, 0.83}, {8.8, 1.06, 1.18}, {11.6, 1.24, 1.48}}}};
+       {{0.90, 0.92, 1.11}, {5.75, 0.98, 1.15}, {5.43, 1.16, 1.36}, {8.40, 1.45, 1.60}}}};
   return us[bits == 8][unit >> 1];
 }
 
@@ -292,7 +296,7 @@ inline WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int bits, int cus,
   const int64_t nu = K / (64 * unit);
   const int bms[4] = {64, 128, 192, 256};
   const WideTileUs* us = wide_tile_us(bits, unit);
-  const double sum_us = unit == 4 ? 3.0 : 6.0;
+  const double sum_us = bits == 4 && unit == 4 ? 3.0 : 6.0;
   WidePlan best;
   bool first = true;
   for (int sp = 1; sp <= max_splits; ++sp) {

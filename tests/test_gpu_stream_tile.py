@@ -62,6 +62,7 @@ TALL = [
     (70, 8200, 2880, 4, 32, BF16, 128, 1, True),      # eleven fours and one, split
     (70, 40007, 384, 4, 64, BF16, 128, 2, False),
     (70, 8200, 2944, 8, 128, BF16, 128, 2, True),
+    (200, 17413, 512, 8, 32, F16, 128, 4, False),
     (200, 17408, 512, 4, 64, F16, 128, 4, False),
     (70, 8200, 4096, 4, 32, BF16, 128, 4, True),
     (450, 17413, 64, 4, 64, BF16, 192, 1, False),     # one step
@@ -77,6 +78,7 @@ TALL = [
     (600, 17408, 384, 4, 128, F16, 256, 2, False),
     (200, 17413, 4224, 8, 64, BF16, 256, 2, True),
     (600, 17413, 512, 4, 64, BF16, 256, 4, False),
+    (600, 17408, 512, 8, 64, F16, 256, 4, False),
     (200, 17408, 5120, 4, 128, BF16, 256, 4, True),
 ]
 
