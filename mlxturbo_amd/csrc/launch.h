@@ -348,19 +348,6 @@ inline int skinny_shared_x_rows(int64_t N, int64_t K, int bits, int gs, int cus)
   return 16;
 }
 
-// Whether 5-8 rows run the shared-x launch with x resident in LDS (the
-// condition of qmv.cuh's launcher restated): m rows of x padded to whole
-// steps plus the three groups' scale copies within the launch's dynamic LDS
-// (kQmvShxLdsMax: the CU's 160 KiB less the static reduction buffers).
-inline bool skinny_resident_x_fits(int64_t m, int64_t K, int bits, int gs) {
-  const int64_t stepk = 4 * (int64_t)gs * ((bits == 4 && gs == 32) ? 2 : 1);
-  const int64_t G = K / gs, stepg = stepk / gs;
-  const int64_t nsteps = (G + stepg - 1) / stepg;
-  const int64_t xres = m * (2 * nsteps * stepk + 16);
-  const int64_t sb = 6 * 2 * 16 * (2 * G + 16);                      // 3 groups x 2 tiles
-  return xres + sb <= 160 * 1024 - 3 * 4 * 2 * 64 * 16;
-}
-
 // K slices (the waves of the one-workgroup launch, 8 on matrices of fewer
 // than 640 16-row tiles) that a skinny launch of m rows runs on separate
 // workgroups (qmv.cuh qmv_split_kernel), or 0: 5-64 rows (16, 32 or 64
@@ -390,51 +377,62 @@ inline size_t skinny_split_bytes(int64_t M, int64_t N, int64_t K, int bits, int 
   return (size_t)most * N * 8 * sizeof(float);
 }
 
-// Wide tile or skinny launches for M > 16 rows.  Up to 64 rows stay on the
-// skinny family wherever it takes them in launches of 32 (shared x) or 64
-// rows (split K slices): there every 16 rows have the bits of their own
-// 16-row call, which verify widths rely on.  Elsewhere the cheaper by a model
-// fitted to measurements: skinny launches take about 3 us plus the weight
-// bytes at 3.6 TB/s for one row, x1.15 for 2-4 rows, x1.4 for 5-8, x1.65 for
-// 9-16; on matrices of 640+ row tiles and 48+ rows per CU (the shared-x
-// workgroups of 5-16 rows) x1.35 for 5-8 and x1.42 for 9-16 (K=5120 N=17408:
-// 20.7 and 21.8 us against 15.4 for the one-row model), and 17-32 rows there
-// in one launch at x1.5 (two 16-row A tiles per weight fragment: M=17/24/32
-// 22.0/21.6/21.1 us, one process); the wide tile by wide_plan (K=5120 N=17408:
-// M=96 from the third row of tiles on, 40 us at 128 rows against 66 in 32-row
-// launches).  split_ok: a workspace is available for K splits.  row_identity
-// (mq_set_row_identity): up to 32 rows on the skinny family for every matrix,
-// whose rows then have the bits of a one-row call.
+// Time of one skinny launch of m rows by a model fitted to 1750 calls of 17-128
+// rows (500 matrices of K=512 .. 17408, N=512 .. 151936; the calls' times within
+// 13%, rms): us per launch, per MB of 4-bit codes (8-bit codes stream faster:
+// 0.72 of it per MB) and per million outputs, which weigh at short K (K=512
+// N=36000 M=48, 8 bits, two launches: 43 us where the weights say 10).
+struct SkinnyUs {
+  double launch, mb, out;
+};
+
+inline double skinny_us(int64_t m, int64_t N, int64_t K, int bits, int gs, int sx, bool split) {
+  const bool long_steps = 4 * gs * ((bits == 4 && gs == 32) ? 2 : 1) > 256;
+  const SkinnyUs c = split ? (m > 32   ? SkinnyUs{7.54, 0.53, 13.6}      // and the sum kernel
+                              : m > 16 ? SkinnyUs{6.40, 0.42, 15.4}
+                                       : SkinnyUs{6.45, 0.31, 0.0})
+                     : m > 16           ? SkinnyUs{6.32, 0.37, 5.1}      // two 16-row A tiles
+                     : m > 4 && sx > 0  ? SkinnyUs{3.00, 0.27, 11.8}     // shared x
+                     : m > 8            ? (long_steps ? SkinnyUs{3.53, 0.56, 6.7}   // x unstaged
+                                                      : SkinnyUs{2.94, 0.36, 10.1})
+                     : m > 4            ? SkinnyUs{3.19, 0.36, 14.9}
+                                        : SkinnyUs{3.36, 0.29, 22.7};
+  const double mb = (double)N * (double)K * bits / 8.0e6 * (bits == 8 ? 0.72 : 1.0);
+  return c.launch + c.mb * mb + c.out * (double)m * (double)N / 1.0e6;
+}
+
+// Wide tile or skinny launches for M > 16 rows: the cheaper by the models
+// (skinny_us, wide_plan).  Over 1750 calls of 17-128 rows it is within 2% of the
+// faster one in the geometric mean.
+//
+// Up to 64 rows the skinny family keeps, where it takes them in launches of 32
+// (shared x) or 64 rows (split K slices), the bits of every 16 rows' own call:
+// there the wide tile is priced at no less than its weights at 0.8 TB/s (8-bit
+// ones 1.2 on the shared-x matrices, 0.9 on the narrow ones), about half the
+// rate it reaches, so that it takes over only where it saves about a third (K=1024 N=36000 M=64 14 us against 37; K=5120 N=17408
+// M=64 stays, 30 against 46).  row_identity (mq_set_row_identity): up to 32
+// rows on the skinny family for every matrix, whose rows then have the bits of
+// a one-row call.  split_ok: a workspace is available for K splits.
 inline bool wide_route(int64_t M, int64_t N, int64_t K, int bits, int gs, int cus, bool split_ok,
                        bool row_identity) {
   if (!wide_eligible(M, N, K, bits, gs) || (row_identity && M <= 32)) return false;
   const int sx = skinny_shared_x_rows(N, K, bits, gs, cus);
-  if (M <= 64 && (sx == 32 || (split_ok && skinny_split_slices(M, N, K, bits, gs)))) return false;
-  const double wbytes = (double)N * (double)K * bits / 8.0;
-  const double wide_us = wide_plan(M, N, K, bits, cus, split_ok ? 16 : 1).cost_us;
-  const double one = 3.0 + wbytes / 3.6e6;
-  const bool shared_x = sx > 0;
-  double skinny_us = 0.0;
+  double wide_us = wide_plan(M, N, K, bits, cus, split_ok ? 16 : 1).cost_us;
+  if (M <= 64 && (sx == 32 || (split_ok && skinny_split_slices(M, N, K, bits, gs)))) {
+    const double tbs = bits == 4 ? 0.8 : sx == 32 ? 1.2 : 0.9;
+    const double least = (double)N * (double)K * bits / (8.0e6 * tbs);
+    if (wide_us < least) wide_us = least;
+  }
+  double skinny = 0.0;
   for (int64_t m0 = 0, step = 16; m0 < M; m0 += step) {
     // with the workspace, 5-64 rows on matrices of few tiles run as one
-    // split launch (K=17408 N=5120: 16 / 32 / 64 rows 21.7 / 26.0-26.6 /
-    // 35.2 us = 1.4 / 1.7 / 2.3 x one; from 96 rows the wide tile, 55.6 us)
+    // split launch
     const int64_t ms = M - m0 < 64 ? M - m0 : 64;
-    if (split_ok && skinny_split_slices(ms, N, K, bits, gs)) {
-      step = ms;
-      skinny_us += one * (ms > 32 ? 2.3 : ms > 16 ? 1.7 : 1.4);
-      continue;
-    }
-    step = sx == 32 && M - m0 > 16 ? 32 : 16;
-    const int64_t m = M - m0 < step ? M - m0 : step;
-    skinny_us += one * (m > 16   ? 1.5
-                        : m > 8  ? (shared_x ? 1.42 : 1.65)
-                        : m > 4  ? (shared_x && skinny_resident_x_fits(m, K, bits, gs) ? 1.35
-                                                                                       : 1.4)
-                        : m > 1  ? 1.15
-                                 : 1.0);
+    const bool split = split_ok && skinny_split_slices(ms, N, K, bits, gs);
+    step = split ? ms : sx == 32 && M - m0 > 16 ? 32 : 16;
+    skinny += skinny_us(M - m0 < step ? M - m0 : step, N, K, bits, gs, sx, split);
   }
-  return wide_us < skinny_us;
+  return wide_us < skinny;
 }
 
 // Workspace bytes of quantized_matmul (K splits of the wide kernel or of the

@@ -17,12 +17,12 @@ Mirrors mlxturbo/kernels/dispatch.py on torch modules:
 
 On MI355X every route is a HIP kernel of this library: ``stock`` is
 :func:`mlxturbo_amd.quantized_matmul` with the library's own width choice
-(the one-row quad kernel, the skinny streaming kernel for 2..32 rows, and
-above that 32- or 16-row skinny launches or the MFMA tile kernel, whichever
-the library's per-geometry cost model prices lower); ``skinny`` and
-``wide`` name the two families.  At K=5120, N=17408 one skinny launch of
-16 rows costs ~21 us and of 32 rows ~23 us, while the MFMA tile kernel does
-96 rows in ~53 us and 512 rows in ~112 us.
+(the one-row quad kernel, the skinny streaming kernel for 2..16 rows, and
+above that skinny launches or the MFMA tile kernel, as the library's
+per-geometry cost model prices them); ``skinny`` and ``wide`` name the two
+families.  At K=5120, N=17408 one skinny launch of 16 rows costs ~21 us and of
+32 rows ~23 us, while the MFMA tile kernel does 96 rows in ~36 us and 512 rows
+in ~89 us.
 """
 
 from __future__ import annotations
@@ -51,9 +51,8 @@ def _row() -> tuple[str, ...]:
 
 # The reference's measured production geometries (dispatch.py:59-68).  Its
 # rows choose among Metal kernels per M; here the per-geometry choice is the
-# library's own cost model (csrc/launch.h wide_route / wide_plan: skinny
-# launch time 3 us + weight bytes at 3.6 TB/s times a factor per row count,
-# wide tile time per round of workgroups, each constant measured on MI355X),
+# library's own cost model (csrc/launch.h wide_route: skinny launches by
+# skinny_us, wide tiles by wide_plan, each constant measured on MI355X),
 # which every call consults, so the default rows only name the streaming
 # kernels at M = 1..16 (what the model picks there on every geometry) and a
 # row is where a caller forces 16-row launches above 16 rows ("skinny").

@@ -488,11 +488,12 @@ def test_skinny_long_k_many_rows(M):
                                       ((5120, 17408), 40), ((5120, 17408), 64),
                                       ((17408, 5120), 17), ((17408, 5120), 24)])
 def test_skinny_launches_above_16_rows(cfg2_weights, shape, M):
-    """Widths where the wide tile would stream its weights at ~0.9 TB/s run
-    as skinny launches: on the tall matrix (48+ rows per CU) up to 32 rows in
-    one launch whose wave groups multiply each weight fragment with two
-    16-row A tiles, on the narrow one 16 rows per launch.  Each block of 16
-    rows is bit-identical to a call of those rows alone (the same K split),
+    """Widths that keep the bits of every 16 rows' own call, where the wide
+    tile does not save a third, run as skinny launches: on the tall matrix
+    (48+ rows per CU) up to 32 rows in one launch whose wave groups multiply
+    each weight fragment with two 16-row A tiles, on the narrow one up to 64
+    rows, the K slices on separate workgroups.  Each block of 16 rows is
+    bit-identical to a call of those rows alone (the same K split),
     and the whole matches the oracle on sampled columns."""
     K, N = shape
     w, s, b, deq, dev = cfg2_weights[shape]
@@ -558,10 +559,10 @@ def test_wide_split_k_narrow_matrix(cfg2_weights, M):
 @pytest.mark.parametrize("M", [40, 100, 300, 600, 512, 1100, 2048, 8192])
 def test_config3_wide(cfg2_weights, M):
     """Prefill widths through the MFMA tile kernel, full size; the oracle checks
-    64 sampled rows x 512 sampled columns.  M=40 runs as 16-row skinny
-    launches; on 256 CUs 100 / 300 / 600 / 8192 pick tile heights 64 / 128 /
-    256 / 256 and 512 / 1100 / 2048 pick 192, all but 8192 with a ragged last
-    row tile."""
+    64 sampled rows x 512 sampled columns.  M=40 runs as skinny launches of
+    32 rows; on 256 CUs 100 / 300 pick tiles of 128 rows (100 in three K
+    splits), 600 / 8192 of 256 and 512 / 1100 / 2048 of 192, all but 8192 with
+    a ragged last row tile."""
     K, N = 5120, 17408
     w, s, b, deq, dev = cfg2_weights[(K, N)]
     rng = np.random.default_rng(300 + M)
@@ -822,9 +823,9 @@ def test_gather_prefill_size_classes(M, bits, gs, sort):
                                              (4, 32, "float16", 2048), (8, 64, "bfloat16", 2048),
                                              (4, 64, "bfloat16", 512), (8, 32, "float16", 512)])
 def test_gather_prefill_scale_blocks(bits, gs, dtype, K):
-    """K / gs a multiple of 8: the grouped tiles (64/128-row wide tiles past
-    K=2048, the thin kernel with 8 waves at K=2048 and 4 at K=512) read
-    scales and biases in 16-byte blocks of 8 groups, one load per block
+    """K / gs a multiple of 8: the grouped tiles past K=2048 and the thin kernel
+    of 4-bit banks read scales and biases in 16-byte blocks of 8 groups, one
+    load per block, the thin kernel of 8-bit banks those of four k-steps
     (group 32: two groups per step, the group index differs across a row's
     chunks; group 128: per-step loads, the block would span 16 steps).
     Ragged N, zipf routing, full oracle."""
@@ -882,7 +883,7 @@ def test_gather_sorted_prep_matches_counting_sort(T, top, M, K):
     kernel's scan path (identity order); the same pairs shuffled take the
     counting sort.  Per-pair rows must be bit-identical, and match the
     oracle.  Covers the streaming kernel with prep tables (P*M < 1024), the
-    thin kernel with 4 and 8 waves and the wide grouped kernels, runs longer
+    thin kernel of 4-bit banks and the wide grouped kernels, runs longer
     than a segment."""
     rng = np.random.default_rng(T + top + M + K)
     E, N = 24, 160

@@ -39,3 +39,20 @@ def test_wide_heights_are_planned():
         assert r == (1, c[6], r[2], c[7]) and (r[2] > 1) == c[8], (c, r)
     assert {(r[0]) for r in routes([(*c, 0, 0) for c in cases])} == {1}
     assert {c[6:8] for c in TALL} == set(itertools.product([128, 192, 256], [1, 2, 4]))
+
+
+@pytest.mark.parametrize("M, N, K, bits, gs, wide", [
+    (48, 36000, 512, 8, 64, 1),      # 12.5 us against 43.3
+    (64, 8192, 512, 4, 64, 1),       # 8.3 against 18.4
+    (64, 36000, 1024, 4, 64, 1),     # 13.6 against 36.7
+    (64, 12288, 1536, 8, 64, 1),     # 20.6 against 38.7
+    (80, 17408, 2880, 8, 64, 1),     # 34.7 against 94
+    (32, 2050, 640, 8, 64, 0),       # 12.1 against 7.5
+    (24, 2050, 576, 4, 64, 0),       # 9.1 against 6.2
+    (64, 17408, 5120, 4, 64, 0),     # bits of 16-row calls: less than a third to gain
+    (64, 5120, 17408, 4, 64, 0),
+])
+def test_route_of_few_rows(M, N, K, bits, gs, wide):
+    """Calls where one family is far slower (wide tile against skinny launches,
+    measured)."""
+    assert routes([(M, N, K, bits, gs, 1, 0)])[0][0] == wide
