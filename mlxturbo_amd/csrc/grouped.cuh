@@ -125,7 +125,7 @@ __device__ __forceinline__ void thin_tile(
   };
   // Scales and biases in 16-byte blocks of 8 groups, one load per block,
   // when K / GS is a multiple of 8 and the arrays are 16-byte aligned (the
-  // scheme and its measurements are those of wide_tile's FRESH tiles): the
+  // scheme and its measurements are those of wide_tile's blocks): the
   // loop below is unrolled over a block so each block load and group index
   // is a compile-time position.
   constexpr int SPB = GS / 8;                   // 64-code steps per block

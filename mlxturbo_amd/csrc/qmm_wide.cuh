@@ -36,19 +36,17 @@ constexpr int kWideLD = kWideBK + 8;  // LDS row stride in 16-bit elements (144 
 template <int BM>
 constexpr size_t wide_lds_bytes() { return 2 * (size_t)(BM + kWideBN) * kWideLD * 2; }
 
-// One BM x 256 output tile over k-steps kt0 .. kt0 + nkl - 1 (64 codes each).
+// One BM x 256 output tile over all K / 64 k-steps of 64 codes.
 // x rows come from xrsrc at per-row byte offsets xrow_off(r) (past the range
 // for rows that do not exist); w / scales / biases point at the tile's first
 // weight row, of which nrows (<= 256) exist; store(r, c, v) receives the
 // float sum of row r, tile column c (< nrows).
-// FRESH: the caller's tiles do not share weight tiles through L2 (grouped
-// segments), which enables per-block scale loads below.
-template <int DT, int BITS, int GS, int BM, class XRowOff, class Store, bool FRESH = false>
+template <int DT, int BITS, int GS, int BM, class XRowOff, class Store>
 __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff xrow_off,
                                           const uint32_t* __restrict__ w,
                                           const uint16_t* __restrict__ scales,
                                           const uint16_t* __restrict__ biases, int nrows, int K,
-                                          int kt0, int nkl, Store store, uint16_t* wide_smem) {
+                                          Store store, uint16_t* wide_smem) {
   constexpr int BN = kWideBN, BK = kWideBK, LD = kWideLD, NT = kWideNT;
   constexpr int WGM = BM == 256 ? 4 : 2;        // waves along M
   constexpr int WGN = 8 / WGM;                  // waves along N
@@ -72,7 +70,7 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
   const int wm = wave / WGN, wn = wave % WGN;
   const int64_t Kw = (int64_t)K * BITS / 32;
   const int G = K / GS;
-  const int nk = nkl;
+  const int nk = K / BK;
 
   // rows past nrows are past the weight range and read zeros
   const auto rwd = wide_rsrc(w, (int64_t)nrows * Kw * 4);
@@ -104,10 +102,9 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
   };
   Set S0, S1;
   bool big = false;   // a scale with |s| >= 2^100 met on the fast route
-  // Scales and biases, 64- and 128-row tiles of weights that no other tile
-  // reads through L2 (on dense tiles it cost 1.5-4%), K / GS a multiple of 8,
-  // both arrays 16-byte aligned and whose k range is whole blocks of SPB
-  // steps: each thread loads the 16-byte block (8 groups) of its rows'
+  // Scales and biases, 64- and 128-row tiles with K / GS a multiple of 8,
+  // both arrays 16-byte aligned and whole blocks of SPB steps in K:
+  // each thread loads the 16-byte block (8 groups) of its rows'
   // scales and biases with the block's first step (ns / nb) and takes it
   // over (cs / cb) when that step is stored, instead of two 2-byte loads
   // per step; the loop is unrolled over a block so every block load and
@@ -115,12 +112,12 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
   // weights (a thin expert) spends ~15% of its time on the per-step
   // requests at K = 2048.
   constexpr int SPB = GS / 8;                   // 64-code steps per block
-  constexpr bool SBLK = FRESH && BM <= 128 && SPB >= 4 && SPB <= 8;
-  const bool sblk = SBLK && G % 8 == 0 && kt0 % SPB == 0 && nk % SPB == 0 &&
+  constexpr bool SBLK = BM <= 128 && SPB >= 4 && SPB <= 8;
+  const bool sblk = SBLK && G % 8 == 0 && nk % SPB == 0 &&
                     ((uintptr_t)scales | (uintptr_t)biases) % 16 == 0;
   u32x4 ns[WPT], nb[WPT], cs[WPT], cb[WPT];
   auto bload = [&](int kt) {
-    const uint32_t bo = 16u * (uint32_t)((kt0 + kt) * BK / GS / 8);
+    const uint32_t bo = 16u * (uint32_t)(kt * BK / GS / 8);
 #pragma unroll
     for (int i = 0; i < WPT; ++i) {
       ns[i] = __builtin_amdgcn_raw_buffer_load_b128(rsd, so[i] + bo, 0, 0);
@@ -128,7 +125,7 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
     }
   };
   auto gload_w = [&](Set& st, int kt) {
-    const int k0 = (kt0 + kt) * BK;
+    const int k0 = kt * BK;
 #pragma unroll
     for (int i = 0; i < XPT; ++i)
       st.xa[i] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, xo[i], k0 * 2, 0);
@@ -137,7 +134,7 @@ __device__ __forceinline__ void wide_tile(__amdgpu_buffer_rsrc_t xrsrc, XRowOff 
       st.wv[i] = __builtin_amdgcn_raw_buffer_load_b128(rwd, wo[i], k0 * BITS / 8, 0);
   };
   auto gload = [&](Set& st, int kt) {
-    const int k0 = (kt0 + kt) * BK;
+    const int k0 = kt * BK;
 #pragma unroll
     for (int i = 0; i < XPT; ++i)
       st.xa[i] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, xo[i], k0 * 2, 0);
@@ -353,9 +350,8 @@ __device__ __forceinline__ void grouped_body(
     const int o = s_orow[r];
     if (o >= 0) ot[(int64_t)o * N + c] = T16<DT>::round1(v);
   };
-  wide_tile<DT, BITS, GS, BM, decltype(xrow_off), decltype(store), true>(
-      xr, xrow_off, w + wrow * K * BITS / 32, scales + wrow * G, biases + wrow * G, ncols, K, 0,
-      K / kWideBK, store, wide_smem);
+  wide_tile<DT, BITS, GS, BM>(xr, xrow_off, w + wrow * K * BITS / 32, scales + wrow * G,
+                              biases + wrow * G, ncols, K, store, wide_smem);
 }
 
 // Expert-grouped tiles of one height over the prep tables' size class cls:
