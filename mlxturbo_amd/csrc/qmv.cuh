@@ -107,15 +107,19 @@ struct QmvGeom {
   static_assert(NSV == 2 || NSV % 4 == 0, "scale vector must be 8 bytes or whole 16-byte loads");
 };
 
-// Bytes that the loads of step t may read from that step's start in a tile's
-// first row (rows of row_bytes, step_bytes of each per step): to the end of the
-// step in the tile's last row, and of the ragged step (tail) to the end of that
-// row, where the matrix may end and mapped memory with it.
+// Bytes that the loads of a whole step may read from the step's start in a
+// tile's first row (rows of row_bytes, step_bytes of each per step): to the end
+// of the step in the tile's last row.
 __host__ __device__ inline uint32_t qmv_step_bytes(int rows, uint32_t row_bytes,
-                                                   uint32_t step_bytes, int t, bool tail) {
-  if (rows <= 0) return 0u;
-  return (uint32_t)(rows - 1) * row_bytes +
-         (tail ? row_bytes - (uint32_t)t * step_bytes : step_bytes);
+                                                   uint32_t step_bytes) {
+  return rows > 0 ? (uint32_t)(rows - 1) * row_bytes + step_bytes : 0u;
+}
+
+// Bytes by which step t ends past its row, which its loads must leave out: the
+// matrix may end with that row, and mapped memory with it.
+__host__ __device__ inline uint32_t qmv_tail_excess(uint32_t row_bytes, uint32_t step_bytes,
+                                                    int t) {
+  return (uint32_t)(t + 1) * step_bytes - row_bytes;
 }
 
 // Launch geometry of the skinny kernel for one (bits, group_size): groups per
@@ -309,6 +313,13 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
   const uint32_t rowB = (uint32_t)K * BITS / 8;
   const int G = K / GS;
   const uint32_t sRowB = (uint32_t)G * 2;
+  uint32_t w_nrec[TJ], s_nrec[TJ];             // of a whole step
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    const int rj = tl.rows[j];
+    w_nrec[j] = qmv_step_bytes(rj, rowB, STEPB);
+    s_nrec[j] = qmv_step_bytes(rj, sRowB, STEPG * 2);
+  }
   const uint32_t wofs = (uint32_t)r * rowB + (uint32_t)c * 16;
   const uint32_t sofs = (uint32_t)r * sRowB;
   // scale of load L: half ((4 L + c) >> SH) & 3 of dword pair ((4 L) >> SH) >> 2
@@ -355,7 +366,7 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     xvo[q] = (m < M && xpi[q] >= 0) ? (uint32_t)(src.xoff(m) + xpk[q]) * 2u : 0x80000000u;
   }
 
-  // tail: the ragged step, whose rows end inside it (qmv_step_bytes); its
+  // tail: the ragged step, whose rows end inside it (qmv_tail_excess); its
   // scales are read one by one, as no wider load is sure to end where they do
   auto load = [&](Stage& s, int t, bool live, bool tail = false) {
     if constexpr (XM > 0 && !XRES) {
@@ -368,7 +379,8 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     }
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
-      const uint32_t wn = qmv_step_bytes(tl.rows[j], rowB, STEPB, t, tail);
+      uint32_t wn = w_nrec[j];
+      if (tail && wn) wn -= qmv_tail_excess(rowB, STEPB, t);
       const auto rw = make_rsrc(tl.w[j] + (int64_t)t * STEPB, live ? wn : 0u);
 #pragma unroll
       for (int L = 0; L < NL; ++L)
@@ -377,7 +389,8 @@ __device__ __forceinline__ void qmv_tile(const QmvTiles<TJ>& tl, int M, int K, c
     if constexpr (!SBL) {
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        const uint32_t sn = qmv_step_bytes(tl.rows[j], sRowB, STEPG * 2, t, tail);
+        uint32_t sn = s_nrec[j];
+        if (tail && sn) sn -= qmv_tail_excess(sRowB, STEPG * 2, t);
         const auto rs = make_rsrc(tl.s[j] + (int64_t)t * STEPG * 2, live ? sn : 0u);
         const auto rb = make_rsrc(tl.b[j] + (int64_t)t * STEPG * 2, live ? sn : 0u);
         if (tail) {

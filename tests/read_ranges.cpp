@@ -27,14 +27,14 @@ void skinny(int64_t K, int64_t N, int64_t E, bool tails, bool scales) {
   using Gm = mq::QmvGeom<BITS, GS, mq::QmvConf<BITS, GS>::GPL>;
   const int64_t G = K / GS, row = scales ? 2 * G : K * BITS / 8;
   const int step = scales ? 2 * Gm::STEPG : Gm::STEPB;
-  const int full = (int)(G / Gm::STEPG), n = (int)((G + Gm::STEPG - 1) / Gm::STEPG);
+  const int full = (int)(G / Gm::STEPG), steps = (int)((G + Gm::STEPG - 1) / Gm::STEPG);
   for (int64_t e : {(int64_t)0, E - 1})
     for (int64_t n0 = 0; n0 < N; n0 += 16)
-      for (int t = 0; t < n; ++t)
-        span((e * N + n0) * row + (int64_t)t * step,
-             mq::qmv_step_bytes((int)std::min<int64_t>(16, N - n0), (uint32_t)row, step, t,
-                                tails && t >= full),
-             E * N * row);
+      for (int t = 0; t < steps; ++t) {
+        uint32_t n = mq::qmv_step_bytes((int)std::min<int64_t>(16, N - n0), (uint32_t)row, step);
+        if (tails && t >= full) n -= mq::qmv_tail_excess((uint32_t)row, step, t);
+        span((e * N + n0) * row + (int64_t)t * step, n, E * N * row);
+      }
 }
 
 // One-row kernel: descriptors of a quad's rows and of the whole scale array.
