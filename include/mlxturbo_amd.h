@@ -60,11 +60,11 @@ uint64_t mq_launch_count(void);
  * wide tile where that is the cheaper: each row is within the output
  * tolerance of all of them, not bit-identical to the same row computed in
  * a call of another width.  With on != 0, calls of 1 to 32 rows all run the
- * 2..32-row kernel family, so a row's result does not depend on how many of
- * these rows the call has
- * (decode vs. speculative verify).  The reference keeps this property with
- * its opt-in small-M route: rows of an M = 2..8 call bit-identical to the
- * M = 1 call (kernels/qmv_small_m.py:289-307, dispatch.py:337-347).
+ * 2..32-row kernel family, so a row's result does not depend on which of
+ * these row counts the call has (decode vs. speculative verify).  The
+ * reference keeps this property with its opt-in small-M route: rows of an
+ * M = 2..8 call bit-identical to the M = 1 call
+ * (kernels/qmv_small_m.py:289-307, dispatch.py:337-347).
  * Returns the previous setting.  Not for calls running concurrently with a
  * change of the setting; workspaces are to be sized under the setting that
  * the call runs under.
@@ -148,9 +148,10 @@ size_t mq_quantized_matmul_workspace_size(int64_t M, int64_t N, int64_t K, int g
  * kernel (same results up to the order of the float sums), and 5-64 rows on
  * matrices of fewer than 640 16-row tiles run their K slices on separate
  * workgroups and add them in a second kernel (every 16 rows get the bits of
- * a 16-row call without the workspace).  Replaces the
- * same mx.quantized_matmul call as mq_quantized_matmul; calls sharing a
- * workspace must be ordered (one stream).
+ * a 16-row call without the workspace; more than 16 rows take the wide kernel
+ * instead where it saves about a third, at short K).  Replaces the same
+ * mx.quantized_matmul call as mq_quantized_matmul; calls sharing a workspace
+ * must be ordered (one stream).
  */
 int mq_quantized_matmul_ws(const void* x, const uint32_t* w, const void* scales,
                            const void* biases, void* out, int64_t M, int64_t N, int64_t K,
