@@ -1,9 +1,9 @@
 """Build ``libmlxturbo_amd.so`` in-tree with hipcc for gfx950.
 
 Usage: ``python -m mlxturbo_amd.build``.  The library is plain C ABI over HIP
-(no torch headers): ``csrc/abi.hip`` (argument checks and routing) plus
-``csrc/inst.hip`` compiled once per (dtype, bits) pair, in parallel, then
-linked into one shared object.
+(no torch headers): ``csrc/abi.hip`` (argument checks and routing) plus the
+kernels' units, compiled once per (dtype, bits) pair or per pair and group
+size, in parallel, then linked into one shared object.
 """
 
 from __future__ import annotations
@@ -50,8 +50,9 @@ UNITS = [("abi.hip", []), ("formats.hip", []), ("prep.hip", []), ("route.hip", [
     for glu in ([], ["-DMQ_INST_GLU"]) for dt in (0, 1) for bits in (4, 8)
 ] + [
     # the wide kernel's instruction order (dense.hip)
-    ("dense.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}", "-fno-slp-vectorize"])
-    for dt in (0, 1) for bits in (4, 8)
+    ("dense.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}", f"-DMQ_INST_GS={gs}",
+                   "-fno-slp-vectorize"])
+    for dt in (0, 1) for bits in (4, 8) for gs in (32, 64, 128)
 ] + [
     # the quad kernel keeps its MFMA accumulators in VGPRs (qmv_quad.cuh)
     ("quad.hip", [f"-DMQ_INST_DT={dt}", f"-DMQ_INST_BITS={bits}", "-mllvm",
